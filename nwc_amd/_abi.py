@@ -41,6 +41,10 @@ SIGNATURES = {
     "nwc_stream_read": ("i", "ppQpI"),
     "nwc_setup": ("i", ""),
 }
+# entry points for this package alone (nwc_amd/csrc/nwc_private.h), not part of the C ABI
+PRIVATE = {
+    "nwc_tokens": ("i", "pppppppppIppppQQIiI"),
+}
 
 
 def library_path():
@@ -55,7 +59,7 @@ def library_path():
 
 def _bind(path):
     lib = ctypes.CDLL(path)
-    for name, (res, args) in SIGNATURES.items():
+    for name, (res, args) in {**SIGNATURES, **PRIVATE}.items():
         fn = getattr(lib, name)
         fn.restype = _CTYPES[res]
         fn.argtypes = [_CTYPES[a] for a in args]

@@ -2,6 +2,7 @@
 // dispatch to the kernel files.  Argument meaning and return codes follow parda21/NWC csrc/nwc_ops.cu:1045-1192.
 #include "nwc_launch.h"
 #include "nwc_ops.h"
+#include "nwc_private.h"
 
 #include <algorithm>
 #include <atomic>
@@ -54,6 +55,7 @@ bool shape_ok(uint64_t n, uint32_t block, uint32_t K, int elem) {
 // weights (2.85-2.99 code bits per weight) ~405; a 16 x 512 block twice that.  Larger blocks decode from global
 // memory instead.
 constexpr uint32_t kSlotWords0 = 480, kSlotWords1 = 960;
+constexpr uint32_t kLdsPerCu = 160u * 1024u;
 constexpr uint32_t kDynLdsBudget = 48u * 1024u;       // dynamic LDS per workgroup next to the 16 KB decode table
 
 uint32_t slot_words_for(int layout) { return layout == 0 ? kSlotWords0 : layout == 1 ? kSlotWords1 : 0u; }
@@ -571,6 +573,61 @@ extern "C" int nwc_prefill_xbf16(void *stream, const uint8_t *data, const uint32
                             elem_stride(elem)},
                   x, ntok};
     return launch_prefill0(elem_type(elem), prefill_tokens_per_tile(row_tiles, ntok, ncu), p, (hipStream_t)stream);
+}
+
+namespace {
+
+// Small batches (kern_tokens.hip): `parts` workgroups per column block, one workgroup per CU in all (the decode table and
+// the activations are staged once a workgroup), with the waves that their LDS share and their rounds of row groups need;
+// the 13-bit table wherever it is given (the stored LUT's 16 KB less bought no wave that paid for its slow steps).
+constexpr uint32_t kMaxTokens = 64;
+bool plan_tokens(const Shape &f, int elem, uint32_t T, int ncu, bool index, bool seq, TokensPlan &q, TokensArgs &p) {
+    const int layout = elem_layout(elem);
+    const uint32_t units = f.groups(), nt = T <= 16u ? 1u : T <= 32u ? 2u : 4u, stride = elem_stride(elem);
+    if ((layout <= 1 && !index) || f.CB > (uint32_t)ncu) return false;
+    p.parts = std::min(units, (uint32_t)ncu / f.CB);
+    // a block's slot and the 16 bytes read past it, or the usual size of packed streams
+    p.cap = layout == 2 ? 0u : stride ? stride / 4u + 4u : layout ? kSlotWords1s : kSlotWords2;
+    p.Mu = f.Mp;
+    q.seq13 = seq && layout <= 1;
+    const uint32_t table = layout == 2 ? (elem_type(elem) == kElemFp8 ? kLutWords : 4u)
+                                       : q.seq13 ? kSeqTableWords : kLutWords + 4u;
+    const uint32_t xs = nt * 16u * kTokensXRow * 4u, taken = xs + 4u * (table + kTokensOverrun) + 256u;
+    const uint32_t own = 4u * (layout == 0 ? kTokensTileWords + p.cap : layout == 1 ? p.cap : kTokensPatchWords);
+    if (taken + own > kLdsPerCu) return false;
+    const uint32_t fit = std::min(kTokensMaxWaves, (kLdsPerCu - taken) / own);
+    const uint32_t per = (units + p.parts - 1u) / p.parts, rounds = (per + fit - 1u) / fit;
+    const uint32_t W = (per + rounds - 1u) / rounds;
+    q.threads = 64u * W;
+    q.grid = p.parts * f.CB;
+    // layout 1: what a lane may read past the last wave's slot when its half's range ends before the other's
+    q.lds = xs + W * own + (layout == 1 ? kTokensOverrun * 4u : 0u);
+    return true;
+}
+
+}  // namespace
+
+extern "C" int nwc_tokens(void *stream, const uint8_t *data, const uint32_t *bases, const uint8_t *hdr, const uint32_t *tab,
+                          const uint8_t *low, const uint16_t *row_index, const uint32_t *seq_table, const uint16_t *x,
+                          uint32_t ldx, const uint16_t *bias, const float *scale, uint16_t *y, void *ws, uint64_t ws_bytes,
+                          uint64_t n, uint32_t K, int elem, uint32_t ntok) {
+    if (!shape_ok(n, kBlock, K, elem) || ntok < 2 || ntok > kMaxTokens || ldx < K) return -1;
+    const int ncu = current_cus();
+    if (ncu <= 0) return (int)hipErrorNoDevice;
+    const int layout = elem_layout(elem);
+    const Shape f((uint32_t)(n / K), K, layout);
+    TokensPlan q;
+    TokensArgs p{};
+    if (!plan_tokens(f, elem, ntok, ncu, row_index != nullptr, seq_table != nullptr, q, p)) return -1;
+    if (4ull * f.CB * ntok * p.Mu > ws_bytes || ws == nullptr || ((uintptr_t)ws & 15u) != 0) return -1;
+    p.a = BlockArgs{data, bases, hdr, tab, low, nullptr, bias, scale, y, layout <= 1 ? row_index : nullptr, f.M, f.K, 1u,
+                    0u, layout <= 1 ? seq_table : nullptr, elem_stride(elem)};
+    p.x = x;
+    p.part = (float *)ws;
+    p.T = ntok;
+    p.ldx = ldx;
+    p.vec = K % 8u == 0 && ldx % 8u == 0 && ((uintptr_t)x & 15u) == 0;
+    return launch_tokens(layout, elem_type(elem), q, p, (hipStream_t)stream);
 }
 
 extern "C" int nwc_row_index(void *stream, const uint8_t *data, const uint32_t *bases, const uint8_t *hdr, const uint32_t *tab,

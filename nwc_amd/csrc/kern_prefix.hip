@@ -15,6 +15,7 @@
 // against BF16 activations in registers (fp32 activations: two v_perm_b32 + two FMAs per pair).
 #include "nwc_device.h"
 #include "nwc_launch.h"
+#include "nwc_prefix.h"
 
 namespace nwc {
 
@@ -81,16 +82,6 @@ __device__ __forceinline__ uint4 raw_row(const uint8_t *__restrict__ low, const 
     return ldnt4(low + off);
 }
 
-// Bit position where part j (0-3) of block b starts in lane L's stream: 0 for the first part, else row-index entry
-// j - 1.  The entry is loaded for every part (the first part's load reads entry 0 and drops it): a load inside a branch
-// makes the compiler wait at the branch's end for it and for every request before it, which would hold back the
-// stream copy by a whole round trip.  Callers request it after their other prologue loads (the compiler may read its
-// register as the don't-care high half of a 64-bit multiply-add operand, which would wait for it).
-__device__ __forceinline__ uint32_t part_start(const BlockArgs &a, uint32_t b, uint32_t j, uint32_t L) {
-    const uint32_t v = a.aux[((uint64_t)b * kRowIndexSplits + (j ? j - 1u : 0u)) * kLanes + L];
-    return j ? v : 0u;
-}
-
 // Weights of one window step for the accumulator / dequant output.
 template <int MODE, bool XBF16>
 __device__ __forceinline__ void use_quad(uint32_t e1, uint32_t e2, uint32_t rk, int k, const XRegs<XBF16> &x, float &sum,
@@ -119,61 +110,6 @@ __device__ __forceinline__ void store_row0(const BlockArgs &a, const Shape &f, u
         o[0] = make_uint4(pw[0], pw[1], pw[2], pw[3]);
         o[1] = make_uint4(pw[4], pw[5], pw[6], pw[7]);
     }
-}
-
-// ---- workgroup staging of the streams of a run of consecutive blocks ----
-// The blocks of a workgroup's tile are consecutive in `data`, so a round of H blocks (one per half-wave) is one
-// contiguous byte range: [bases[b_lo], bases[b_hi]) -- for the matrix's last block, its base plus four bytes per header
-// word.  All threads copy it into LDS with 16-byte loads; no half-wave needs its own header scan before the copy.
-// With fixed slots (stride != 0) the range is [b_lo * stride, b_hi * stride) and nothing is read to find it.
-struct Region {
-    uint32_t lo16, n16;         // 16-byte aligned start (byte offset into data), 16-byte chunks
-};
-
-// One past the last stream byte of the matrix (block nb - 1: its base plus four bytes per header word).
-__device__ __forceinline__ uint32_t matrix_end(const BlockArgs &a, uint32_t nb) {
-    const uint32_t *h = (const uint32_t *)(a.hdr + (uint64_t)(nb - 1u) * kHdrBytes);
-    uint32_t words = 0;
-#pragma unroll
-    for (int i = 0; i < (int)kHdrBytes / 4; i++) words = __builtin_amdgcn_udot4(h[i], 0x01010101u, words, false);
-    return a.bases[nb - 1u] + 4u * words;
-}
-
-// Blocks [b_lo, b_hi) plus the 16 bytes the last lane's window reads past its stream (inside the 64 slack bytes that
-// follow the matrix's last block, or the 128 after its last slot).  stride: a.stride (fixed slots) or 0 (bases[]).
-__device__ __forceinline__ Region region_of(const BlockArgs &a, uint32_t b_lo, uint32_t b_hi, uint32_t nb, uint32_t mend,
-                                            uint32_t stride) {
-    Region r;
-    if (stride) {
-        r.lo16 = b_lo * stride;                                 // a multiple of 16
-        r.n16 = ((b_hi > b_lo ? b_hi - b_lo : 0u) * stride + 31u) >> 4;
-        return r;
-    }
-    const uint32_t s = a.bases[b_lo], e = a.bases[min(b_hi, nb - 1u)];
-    r.lo16 = s & ~15u;
-    r.n16 = ((b_hi < nb ? e : mend) + 16u - r.lo16 + 15u) >> 4;
-    return r;
-}
-
-// Four 16-byte chunks per thread cover a region buffer of up to 512 words per half-wave; native vectors keep the
-// words in registers.  Only chunks inside the region are requested (a wave wholly past it issues nothing): the
-// prologue's vector-memory instructions all pass through the CU's address unit, so a workgroup that requested its
-// full four chunks per thread would delay the other workgroup on its CU (o_proj: 9.3 -> 8.7 us).
-struct Bulk {
-    u32x4_t v0, v1, v2, v3;
-};
-__device__ __forceinline__ void bulk_issue(Bulk &B, const uint8_t *__restrict__ data, const Region &r, uint32_t tid, uint32_t nth) {
-    const uint8_t *p = data + r.lo16;
-    if (tid < r.n16) B.v0 = *(const u32x4_t *)(p + 16u * tid);
-    if (tid + nth < r.n16) B.v1 = *(const u32x4_t *)(p + 16u * (tid + nth));
-    if (tid + 2u * nth < r.n16) B.v2 = *(const u32x4_t *)(p + 16u * (tid + 2u * nth));
-    if (tid + 3u * nth < r.n16) B.v3 = *(const u32x4_t *)(p + 16u * (tid + 3u * nth));
-}
-__device__ __forceinline__ void bulk_commit(const Bulk &B, uint32_t *buf, const Region &r, uint32_t tid, uint32_t nth) {
-    if (tid < r.n16) *(u32x4_t *)(buf + 4u * tid) = B.v0;
-    if (tid + nth < r.n16) *(u32x4_t *)(buf + 4u * (tid + nth)) = B.v1;
-    if (tid + 2u * nth < r.n16) *(u32x4_t *)(buf + 4u * (tid + 2u * nth)) = B.v2;
-    if (tid + 3u * nth < r.n16) *(u32x4_t *)(buf + 4u * (tid + 3u * nth)) = B.v3;
 }
 
 // One row of a layout-0 block for one lane (16 weights = four steps of the cursor), dot product with the lane's
@@ -215,23 +151,6 @@ constexpr int kRingD = 8;
 template <int MODE>
 constexpr int ring_depth() { return MODE == kDequant ? kRingD : kRing0; }
 
-// The table entries of one row's 16 weights for one lane (four steps of the cursor; a step that was not fast in some
-// lane is redone code by code by the whole wave), kept apart from their use so that a row can be decoded before its
-// raw bytes have arrived.
-template <int ELEM, class Tab>
-__device__ __forceinline__ void row_codes(Seq<ELEM> &S, const Tab &s, uint32_t (&e1)[4], uint32_t (&e2)[4]) {
-#pragma unroll
-    for (int k = 0; k < 4; k++) {
-        const uint32_t s0 = S.s;
-        const uint32_t *wp0 = S.wp;
-        if (__builtin_expect(__any(S.fast_quad(s, e1[k], e2[k]) >= kSeqSlowTest), 0)) {
-            S.s = s0;
-            S.wp = wp0;
-            S.reload();
-            S.slow_quad(s, e1[k], e2[k]);
-        }
-    }
-}
 // The lane's partial dot product of one row from its entries, raw bytes and activations (token and fp32 modes).
 template <int MODE, bool XBF16>
 __device__ __forceinline__ float row_dot(const uint32_t (&e1)[4], const uint32_t (&e2)[4], const uint4 &rw,
@@ -383,27 +302,6 @@ __device__ __forceinline__ float rowsN_global(const Tab &s, const uint32_t *lane
 //   PIPE = true: two region buffers; while round k decodes, round k + 1's streams, raw rows (four-register ring) and
 //     activations are in flight and round k + 2's bounds and header bytes are read, so after the first round no step
 //     waits on global memory.  One barrier per round publishes the next region.
-// Staging of the decode table: the stored 12-bit LUT, re-encoded (PEEK 12), or the prepared 13-bit table (PEEK 13).
-template <int PEEK> struct TabStage;
-// issue: the first chunks of the decode table; commit: store them; finish: the chunks a small workgroup has left,
-// called after every request that must not wait for the streams (lut_finish says why)
-template <> struct TabStage<kPeek> {
-    LutLoad Q;
-    __device__ __forceinline__ void issue(const BlockArgs &a, uint32_t nth = blockDim.x) { lut_issue(Q, a.lut, nth); }
-    __device__ __forceinline__ void commit(LutLds &s, uint32_t nth = blockDim.x) { lut_commit<kLutSeq>(s, Q, nth); }
-    __device__ __forceinline__ void finish(LutLds &s, const BlockArgs &a, uint32_t nth = blockDim.x) {
-        lut_finish<kLutSeq>(s, a.lut, nth);
-    }
-};
-template <> struct TabStage<kPeekSeq> {
-    SeqLoad Q;
-    __device__ __forceinline__ void issue(const BlockArgs &a, uint32_t nth = blockDim.x) { seq_issue(Q, a.seq, nth); }
-    __device__ __forceinline__ void commit(LutLds13 &s, uint32_t nth = blockDim.x) { seq_commit(s, Q, nth); }
-    __device__ __forceinline__ void finish(LutLds13 &s, const BlockArgs &a, uint32_t nth = blockDim.x) {
-        seq_finish(s, a.seq, nth);
-    }
-};
-
 // nth: the workgroup's threads; flags: which of scale / bias are set (kFinishAll: read the pointers), for the token
 // kernels whose arguments the hardware preloads (k_layout0p, k_layout0t) and which therefore read neither blockDim nor
 // those pointers from memory before their first requests.  rg0: the tile's first row group.  PART: the workgroup
@@ -633,12 +531,6 @@ static void launch_layout0p(const LaunchPlan &p, const BlockArgs &a, hipStream_t
 // Layout 1: lane L = (r = L >> 2, q = L & 3) holds, per 32-column super-chunk, columns 8q..8q+7 of rows r and r+8.
 // Stream positions 4k..4k+3 of a super-chunk are (row r, cols 2k, 2k+1) then (row r+8, cols 2k, 2k+1), so the four
 // codes of one window step pair with raw word k and with activation pair k of the lane's 16-byte x slice.
-template <int ELEM>
-__device__ __forceinline__ uint4 raw_slot1(const uint8_t *__restrict__ p) {
-    if (ELEM == kElemFp8) return expand_nibbles(ldnt2(p));
-    return ldnt4(p);
-}
-
 // One layout-1 block for one lane: returns (row r sum, row r+8 sum) reduced over the lane's quad, or stores the rows.
 template <int ELEM, int MODE, bool XBF16, typename P>
 __device__ __forceinline__ float2 rows1(const LutLds &s, P words, const BlockArgs &a, const Shape &f, const uint8_t *rp,
@@ -735,29 +627,6 @@ __global__ void __launch_bounds__(1024) k_layout1(BlockArgs a) {
 // (SP = 16 / NS half-waves per block; with SP > 1 the row index gives each lane's bit position at super-chunk
 // 4, 8, 12).  Raw super-chunks go through a ring of two registers (chunk s + 2 is requested when chunk s is done).  Partial row sums are kept per (row, column block, part) and summed in a fixed
 // order by the workgroup.
-struct Coord1 {
-    uint32_t g, cb, b, rb, nsc;
-    uint32_t ro;                // byte offset in `low` of the lane's raw bytes of super-chunk 0 of the block
-};
-template <int ELEM>
-__device__ __forceinline__ Coord1 coord1(uint32_t t, uint32_t rg0, const Shape &f, uint32_t L) {
-    constexpr uint32_t RB = ELEM == kElemFp8 ? 8u : 16u;
-    Coord1 c;
-    c.g = t / f.CB;
-    c.cb = t - c.g * f.CB;
-    c.rb = rg0 + c.g;
-    c.b = c.rb * f.CB + c.cb;
-    c.nsc = c.cb == f.CB - 1u ? f.nsl : 16u;
-    c.ro = ((c.rb * f.spr + c.cb * 16u) * kLanes + L) * RB;
-    return c;
-}
-// Raw super-chunk sc of a block; past the block's last super-chunk it re-reads the last, so loads stay unconditional.
-// 32-bit offsets (the plane is below 4 GB: M * K16 < 2^32) keep one address register per load.
-template <int ELEM>
-__device__ __forceinline__ uint4 raw1(const uint8_t *__restrict__ low, const Coord1 &c, uint32_t sc) {
-    constexpr uint32_t RB = ELEM == kElemFp8 ? 8u : 16u;
-    return raw_slot1<ELEM>(low + (c.ro + min(sc, c.nsc - 1u) * (kLanes * RB)));
-}
 // Eight activations from kc as BF16 pairs (fp32 x: rounded to BF16, as the reference's fp32 path does for layouts
 // 1/2).  x holds K32 values, so every coded super-chunk is in bounds.
 template <bool XBF16>

@@ -24,6 +24,25 @@ int launch_gather_prefix(int layout, int elem_t, const GatherArgs &a, hipStream_
 int launch_gather0x(int layout, int elem_t, const GatherArgs &a, const uint16_t *aux, const uint32_t *seq, hipStream_t st);
 // layout-0 token path for ntok (2..4) activation vectors at once (k_layout0_batch); plan from plan_layout0_batch
 int launch_layout0_batch(const LaunchPlan &p, int elem_t, const BlockArgs &a, uint32_t ntok, hipStream_t st);
+// A small batch of tokens on the matrix cores (kern_tokens.hip).
+struct TokensArgs {
+    BlockArgs a;            // out: y BF16 [T x M]; aux: the row index (layout 1); seq: the 13-bit table
+    const uint16_t *x;      // BF16 [T][ldx]
+    float *part;            // sums of each column block [CB][T][Mu]
+    uint32_t T, ldx, Mu;    // Mu: rows of all row groups
+    bool vec;               // K and ldx multiples of 8, x 16-byte aligned
+    uint32_t parts;         // workgroups per column block
+    uint32_t cap;           // LDS words of a block's streams in a wave's share (layouts 0/1)
+};
+struct TokensPlan {
+    uint32_t grid, threads, lds;
+    bool seq13;
+};
+constexpr uint32_t kTokensMaxWaves = 16;
+// LDS words: a token's 512 activations (rows 4 banks apart); of a wave: layout 0's tile of exponent bytes (8 rows), layout 2's super-chunk pair
+constexpr uint32_t kTokensXRow = 260, kTokensTileRow = 132, kTokensTileWords = 8 * kTokensTileRow, kTokensPatchWords = 512;
+constexpr uint32_t kTokensOverrun = 128;   // 7 super-chunks x 16 codes of at most 24 bits, and the cursor's words
+int launch_tokens(int layout, int elem_t, const TokensPlan &q, const TokensArgs &p, hipStream_t st);
 int launch_gather_fixed(int elem_t, const GatherArgs &a, hipStream_t st);
 // layout-0 prefill (k_prefill0): tt tokens per workgroup tile (64, 128, 256 or 512)
 int launch_prefill0(int elem_t, uint32_t tt, const PrefillArgs &p, hipStream_t st);

@@ -2,7 +2,8 @@
 compressed in HBM and multiply through the gfx950 library.
 
     one token (batch 1)  -> fused decode-matvec kernel, weights decoded in registers (nwc_linear_xbf16)
-    several tokens       -> the matrix decompressed into a temporary BF16 buffer, then F.linear (hipBLASLt)
+    2 to 64 tokens       -> decode + matrix cores without a temporary matrix (nwc_linear_xbf16_batch, nwc_tokens)
+    more tokens          -> the matrix decompressed into a temporary BF16 buffer, then F.linear (hipBLASLt)
 
 The public names, arguments, buffer contracts and exceptions are those of the reference bridge (parda21/NWC
 nwc/nwc_torch.py: NWCWeight :126-269, NWCLinear :306-327, NWCEmbedding :330-344, fuse :360-386, convert :389-445,
@@ -49,6 +50,13 @@ ROW_INDEX = os.environ.get("NWC_ROW_INDEX", "1") != "0"   # layouts 0/1: build t
 # temporary BF16 matrix + F.linear
 BATCH_MAX = int(os.environ.get("NWC_BATCH_MAX", "8"))
 BATCH_LAUNCH = 4                                           # vectors per nwc_linear_xbf16_batch launch
+# matrices of at least TOKENS_MIN_WEIGHTS weights: inputs of TOKENS_MIN (layout 0, whose batched kernel is faster below:
+# 19456 x 2560 at two tokens 19 us against 27) or 2 (layouts 1/2) up to TOKENS_MAX tokens go through the matrix-core
+# kernel (nwc_tokens; at 64 tokens 42 us against 70 of the temporary matrix and hipBLASLt on 19456 x 2560, above that
+# F.linear's tiles fill).  Smaller matrices are a few microseconds either way and keep F.linear's bits.
+TOKENS_MIN, TOKENS_MAX_K = 4, 16384
+TOKENS_MAX = min(64, int(os.environ.get("NWC_TOKENS_MAX", "64")))      # 0: never
+TOKENS_MIN_WEIGHTS = 1 << 20
 # more tokens, layout 0: "dequant" (default) decompresses into a temporary BF16 matrix and multiplies it with
 # linear_dequantized (hipBLASLt, or the library's GEMM where that is faster); "fused" runs nwc_prefill_xbf16 (decode
 # into LDS + matrix cores, no temporary matrix; correct, but slower on MI355X at 512 tokens: 19 ms against 8.0 ms
@@ -529,6 +537,24 @@ class NWCWeight:
                  ptr(self.scale), ptr(y[t0]), self.n, self.in_features, self.code, nt)
         return y
 
+    def takes_tokens(self, tokens):
+        """Whether linear_tokens takes an input of this many vectors and is the fastest route for it."""
+        return ((TOKENS_MIN if self.layout == 0 else 2) <= tokens <= TOKENS_MAX and self.n >= TOKENS_MIN_WEIGHTS
+                and self.in_features <= TOKENS_MAX_K and (self.layout == 2 or self.row_index() is not None))
+
+    def linear_tokens(self, x: torch.Tensor, bias) -> torch.Tensor:
+        """A small batch on the matrix cores without a temporary BF16 matrix, any layout: x BF16 [T, in_features], T from
+        2 to 64, -> y BF16 [T, out_features] = scale * (x W^T) + bias, accumulated in fp32 and rounded once."""
+        _need_gpu(self.data)
+        T = x.shape[0]
+        x = x.contiguous()
+        y = torch.empty(T, self.out_features, dtype=torch.bfloat16, device=x.device)
+        work = torch.empty(T * self._n_scratch, dtype=torch.float32, device=x.device)
+        call("nwc_tokens", stream(), *self._streams(), ptr(self.row_index()), ptr(self.seq_table()), ptr(x),
+             self.in_features, ptr(bias), ptr(self.scale), ptr(y), ptr(work), 4 * work.numel(), self.n, self.in_features,
+             self.code, T)
+        return y
+
     def prefill(self, x: torch.Tensor, bias) -> torch.Tensor:
         """Several BF16 tokens at once, layout 0, without a temporary BF16 matrix: x [T, in_features] -> y BF16
         [T, out_features] = x W^T (fp8: times the row scales) + bias, accumulated in fp32 on the matrix cores
@@ -594,12 +620,23 @@ def _bf16_bias(bias, device):
     return nn.Parameter(bias.detach().to(device=device, dtype=torch.bfloat16), requires_grad=False)
 
 
+def _plain(x, device):
+    """x is an ordinary tensor on `device` that nothing but the values of its product is wanted from: no gradient to
+    x, no forward-mode or functorch transform, no dispatch mode, tracing or autocast to another type, all of which
+    F.linear serves and a kernel called by address would pass by."""
+    return (type(x) is torch.Tensor and x.device == device and not (x.requires_grad and torch.is_grad_enabled())
+            and torch._C._functorch.maybe_current_level() is None and torch.autograd.forward_ad._current_level < 0
+            and not torch._C._len_torch_dispatch_stack() and torch._C._get_tracing_state() is None
+            and (not torch.is_autocast_enabled("cuda") or torch.get_autocast_dtype("cuda") == torch.bfloat16))
+
+
 class NWCLinear(nn.Module):
     """nn.Linear over a compressed matrix (elem "bf16" lossless, or "fp8" weight-only).  One BF16 token goes through
-    the fused decode-matvec kernel, up to NWC_BATCH_MAX (8) BF16 tokens of a layout-0 matrix through the batched one
-    (the matrix decoded once per four tokens); anything else through a temporary BF16 matrix and linear_dequantized
-    (hipBLASLt, or the library's split-K GEMM where that is faster), or, with NWC_PREFILL=fused, BF16 tokens of a
-    layout-0 matrix through the fused prefill kernel (NWCWeight.prefill)."""
+    the fused decode-matvec kernel, a few tokens of a layout-0 matrix (up to 3, or NWC_BATCH_MAX where the matrix-core
+    kernel does not take the input) through the batched one (the matrix decoded once per four tokens), up to 64 tokens
+    through the matrix-core kernel (NWCWeight.takes_tokens says which); anything else through a temporary BF16 matrix
+    and linear_dequantized (hipBLASLt, or the library's split-K GEMM where that is faster), or, with
+    NWC_PREFILL=fused, BF16 tokens of a layout-0 matrix through the fused prefill kernel (NWCWeight.prefill)."""
 
     def __init__(self, linear: nn.Linear = None, device="cuda", block=None, w: "NWCWeight" = None, bias=None,
                  elem="bf16"):
@@ -618,6 +655,10 @@ class NWCLinear(nn.Module):
             y = self.w.linear_bf16(x.contiguous().view(-1), self._bias_data())
             return y.view(*x.shape[:-1], self.out_features)
         tokens = x.numel() // self.in_features
+        if (x.dtype == torch.bfloat16 and self.w.takes_tokens(tokens) and x.shape[-1] == self.in_features
+                and PREFILL != "fused" and _plain(x, self.w.data.device)):
+            y = self.w.linear_tokens(x.reshape(tokens, self.in_features), self._bias_data())
+            return y.view(*x.shape[:-1], self.out_features)
         if x.dtype == torch.bfloat16 and self.w.layout == 0 and 1 < tokens <= BATCH_MAX and self.w.K16 <= 16384:
             y = self.w.linear_batch(x.reshape(tokens, self.in_features), self._bias_data())
             return y.view(*x.shape[:-1], self.out_features)
