@@ -76,12 +76,13 @@ HAS_ELEM, HAS_LAYOUT1, HAS_LAYOUT2 = (lib.nwc_info(i) == 1 for i in range(5, 8))
 
 def ptr(t):
     """Device or host address of a tensor (None passes a null pointer)."""
-    return None if t is None else ctypes.c_void_p(t.data_ptr())
+    return None if t is None else t.data_ptr()
 
 
 def stream():
-    """torch's current HIP stream as the ABI's void* stream argument."""
-    return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    """torch's current HIP stream of the current device, as the ABI's void* stream argument (the handle itself: building
+    torch's stream object for every call took 2.8 us of the 11.6 of one token's call)."""
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
 def call(name, *args):

@@ -496,6 +496,16 @@ class NWCWeight:
         x = (F.pad(x, (0, extra)) if extra else x).contiguous()
         return x if x.data_ptr() % 16 == 0 else x.clone()          # the kernels read x in 16-byte pieces
 
+    def _rows16(self, x):
+        """x [T, in_features] as BF16 rows of K16 columns, zero past in_features; x itself where it is that already
+        (the kernels read it in 16-byte pieces)."""
+        if (self.K16 == self.in_features and x.dtype == torch.bfloat16 and x.is_contiguous()
+                and x.data_ptr() % 16 == 0):
+            return x
+        rows = torch.zeros(x.shape[0], self.K16, dtype=torch.bfloat16, device=x.device)
+        rows[:, :self.in_features] = x
+        return rows
+
     def matvec(self, x_f32: torch.Tensor) -> torch.Tensor:
         """fp32 test path: y = W x in fp32 (times the row scale for fp8)."""
         _need_gpu(self.data)
@@ -528,13 +538,12 @@ class NWCWeight:
         if self.layout != 0:
             raise ValueError("linear_batch: layout 0 only")
         T = x.shape[0]
-        xin = torch.zeros(T, self.K16, dtype=torch.bfloat16, device=x.device)
-        xin[:, :self.in_features] = x
+        xin = self._rows16(x)
         y = torch.empty(T, self.out_features, dtype=torch.bfloat16, device=x.device)
         for t0 in range(0, T, BATCH_LAUNCH):
-            nt = min(BATCH_LAUNCH, T - t0)
-            call("nwc_linear_xbf16_batch", stream(), *self._streams(), ptr(self.seq_table()), ptr(xin[t0]), ptr(bias),
-                 ptr(self.scale), ptr(y[t0]), self.n, self.in_features, self.code, nt)
+            call("nwc_linear_xbf16_batch", stream(), *self._streams(), ptr(self.seq_table()),
+                 ptr(xin) + 2 * t0 * self.K16, ptr(bias), ptr(self.scale), ptr(y) + 2 * t0 * self.out_features, self.n,
+                 self.in_features, self.code, min(BATCH_LAUNCH, T - t0))
         return y
 
     def takes_tokens(self, tokens):
@@ -563,12 +572,7 @@ class NWCWeight:
         if self.layout != 0:
             raise ValueError("prefill: layout 0 only")
         T = x.shape[0]
-        if (self.K16 == self.in_features and x.dtype == torch.bfloat16 and x.is_contiguous()
-                and x.data_ptr() % 16 == 0):         # the kernel reads x in 16-byte pieces
-            xin = x
-        else:
-            xin = torch.zeros(T, self.K16, dtype=torch.bfloat16, device=x.device)
-            xin[:, :self.in_features] = x
+        xin = self._rows16(x)
         y = torch.empty(T, self.out_features, dtype=torch.bfloat16, device=x.device)
         call("nwc_prefill_xbf16", stream(), *self._streams(), ptr(self.row_index()), ptr(self.seq_table()), ptr(xin),
              ptr(bias), ptr(self.scale), ptr(y), self.n, self.in_features, self.code, T)
@@ -652,8 +656,7 @@ class NWCLinear(nn.Module):
 
     def forward(self, x):
         if x.dtype == torch.bfloat16 and x.numel() == self.in_features:
-            y = self.w.linear_bf16(x.contiguous().view(-1), self._bias_data())
-            return y.view(*x.shape[:-1], self.out_features)
+            return self.w.linear_bf16(x.reshape(-1), self._bias_data()).view(*x.shape[:-1], self.out_features)
         tokens = x.numel() // self.in_features
         if (x.dtype == torch.bfloat16 and self.w.takes_tokens(tokens) and x.shape[-1] == self.in_features
                 and PREFILL != "fused" and _plain(x, self.w.data.device)):
