@@ -81,8 +81,8 @@ int nwc_linear_bf16(void *stream, const uint8_t *data, const uint32_t *bases, co
                     const uint8_t *low, const float *x, const uint16_t *bias, const float *scale, float *scratch,
                     uint16_t *y, uint64_t n, uint32_t block, uint32_t K, int elem);
 
-/* Token path with x as BF16 for every layout (layout 0: BF16 [K16]; layouts 1/2: BF16 [K32]), otherwise as
- * nwc_linear_bf16.  row_index: the row index from nwc_row_index, or NULL; with it, small matrices decode each block
+/* Token path with x as BF16 [K] for every layout (values past K are not read; K below 16: zero-extended to BF16
+ * [K16], layouts 1/2 [K32]), otherwise as nwc_linear_bf16.  row_index: the row index from nwc_row_index, or NULL; with it, small matrices decode each block
  * on two or four half-waves at once (same results).  seq_table: the 13-bit decode table of layouts 0/1 from
  * nwc_seq_table (device, 8196 words), or NULL; with it fewer decode steps take the slow path (same results).  No counterpart in
  * the reference, whose Python side converts x to fp32 for layout 0 with an extra kernel (nwc_torch.py:238-239);

@@ -353,20 +353,19 @@ bool plan_layout1_budget(const Shape &f, int mode, int ncu, bool index, uint32_t
 // Layouts 1/2: workgroup tile = G whole row groups, one block per half-wave where the LDS budget allows.  Prefer at
 // least two workgroups per CU (small matrices spread over the whole chip), at most 32 blocks (16 waves) per
 // workgroup, and an even block count so both halves of every wave have a block.
-bool plan_blocks(const Shape &f, int layout, int mode, int ncu, bool index, LaunchPlan &p, bool seq = false,
-                 bool fp8 = false) {
+bool plan_blocks(const Shape &f, int layout, int mode, int ncu, bool index, LaunchPlan &p, bool seq = false) {
     if (layout == 0) return plan_layout0(f, mode, ncu, index, seq, p);
     if (layout == 1 && plan_layout1(f, mode, ncu, index, seq, p)) return true;
     if (mode == kRowIndex) return false;
     p = LaunchPlan{};
     p.layout = layout;
     const uint32_t CB = f.CB, groups = f.groups(), slot = slot_words_for(layout);
-    // layout 2, BF16 token path: G = ceil(groups / (2 CUs)) whole row groups per workgroup, each block's 16
+    // layout 2, token path: G = ceil(groups / (2 CUs)) whole row groups per workgroup, each block's 16
     // super-chunks split into four (or two) ranges.  With at most 32 ranges per tile, one half-wave each (7B qkv, o);
     // otherwise four ranges per block go round-robin over 32 half-waves (7B gate_up: 41.2 -> 36.5-36.9 us against one
     // half-wave per block, down 25.9 -> 23.7).  x is staged in LDS as BF16 (the token path of layouts 1/2 always
     // takes BF16 x).
-    if (layout == 2 && !fp8 && mode == kToken) {
+    if (layout == 2 && mode == kToken) {
         const uint32_t G = std::max(1u, (groups + 2u * (uint32_t)ncu - 1u) / (2u * (uint32_t)ncu));
         auto lds_sp = [&](uint32_t sp) { return (f.K16 + 31u) / 32u * 64u + G * f.rows * CB * sp * 4u; };
         auto take = [&](uint32_t sp, uint32_t halves) {
@@ -388,7 +387,7 @@ bool plan_blocks(const Shape &f, int layout, int mode, int ncu, bool index, Laun
     if (G > 1 && ((G * CB) & 1u)) G--;
     // layout 2's token path when the split's partial sums do not fit (whole blocks, one round): at most two
     // workgroups per CU even if a tile then holds more blocks than half-waves
-    if (layout == 2 && !fp8 && mode == kToken && CB < 32u)
+    if (layout == 2 && mode == kToken && CB < 32u)
         G = std::max(G, (groups + 2u * (uint32_t)ncu - 1u) / (2u * (uint32_t)ncu));
     if (G > groups) G = groups;
     if (G == 0) G = 1;
@@ -406,7 +405,7 @@ bool plan_blocks(const Shape &f, int layout, int mode, int ncu, bool index, Laun
     p.threads = 32u * halves;
     p.grid = (groups + G - 1) / G;
     p.lds = lds_of(G, halves);
-    if (layout == 2 && !fp8 && mode == kToken) {        // the single-round kernel with one half-wave per block
+    if (layout == 2 && mode == kToken) {                // the single-round kernel with one half-wave per block
         // (activations staged in LDS and loads four super-chunks ahead: 7B gate_up 47.6 -> 43.6 us, down 27.6 -> 25.9)
         const uint32_t xb = (f.K16 + 31u) / 32u * 64u;
         if (p.lds + xb <= kDynLdsPipe) {
@@ -425,8 +424,7 @@ int run_blocks(int mode, bool xbf16, hipStream_t st, const uint8_t *data, const 
     const int layout = elem_layout(elem), t = elem_type(elem);
     const Shape f((uint32_t)(n / K), K, layout);
     LaunchPlan p;
-    if (!plan_blocks(f, layout, mode, ncu, aux != nullptr && layout <= 1, p, seq != nullptr && layout <= 1 && xbf16,
-                     t == kElemFp8))
+    if (!plan_blocks(f, layout, mode, ncu, aux != nullptr && layout <= 1, p, seq != nullptr && layout <= 1 && xbf16))
         return -1;
     BlockArgs a{data, bases, hdr, tab, low, x, bias, scale, out, aux, f.M, f.K, p.G,
                 layout == 0 || p.split ? p.slot_words : slot_words_for(layout), seq, elem_stride(elem)};
@@ -590,8 +588,7 @@ bool plan_tokens(const Shape &f, int elem, uint32_t T, int ncu, bool index, bool
     p.cap = layout == 2 ? 0u : stride ? stride / 4u + 4u : layout ? kSlotWords1s : kSlotWords2;
     p.Mu = f.Mp;
     q.seq13 = seq && layout <= 1;
-    const uint32_t table = layout == 2 ? (elem_type(elem) == kElemFp8 ? kLutWords : 4u)
-                                       : q.seq13 ? kSeqTableWords : kLutWords + 4u;
+    const uint32_t table = layout == 2 ? 0u : q.seq13 ? kSeqTableWords : kLutWords + 4u;
     const uint32_t xs = nt * 16u * kTokensXRow * 4u, taken = xs + 4u * (table + kTokensOverrun) + 256u;
     const uint32_t own = 4u * (layout == 0 ? kTokensTileWords + p.cap : layout == 1 ? p.cap : kTokensPatchWords);
     if (taken + own > kLdsPerCu) return false;

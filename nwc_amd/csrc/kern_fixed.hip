@@ -12,9 +12,7 @@ namespace nwc {
 
 template <int ELEM, int MODE, bool XBF16>
 __global__ void __launch_bounds__(1024) k_layout2(BlockArgs a) {
-    __shared__ MantLds ms;
     extern __shared__ float part[];
-    if (ELEM == kElemFp8) stage_mant(ms);
     const RankTab tab{a.lut[0], a.lut[1], a.lut[2], a.lut[3]};
     constexpr uint32_t esz = ELEM == kElemFp8 ? 2u : 3u;
     const uint32_t tid = threadIdx.x, L = tid & 31, r = L >> 2, q = L & 3;
@@ -44,7 +42,8 @@ __global__ void __launch_bounds__(1024) k_layout2(BlockArgs a) {
                     if (row0 + r + 8 < f.M) *(uint4 *)(o + (uint64_t)(r + 8) * f.K16) = make_uint4(qq[0], qq[1], qq[2], qq[3]);
                 }
             } else if (XBF16) {
-                const uint4 xv = *(const uint4 *)((const uint16_t *)a.x + kc);
+                const uint4 xv = kc + 8u <= f.K || f.K < 16u ? *(const uint4 *)((const uint16_t *)a.x + kc)
+                                                             : x8_tail((const uint16_t *)a.x, kc, f.K);
 #pragma unroll
                 for (int k = 0; k < 4; k++) {
                     accA = dot2_bf16(p[k], u4_get(xv, k), accA);
@@ -70,11 +69,11 @@ __global__ void __launch_bounds__(1024) k_layout2(BlockArgs a) {
                 const uint32_t c2 = ldnt1((pp + 2 * kLanes * 4));
                 uint32_t p[4], qq[4];
                 const uint2 n0 = ldnt2((np + (uint64_t)(2 * sp) * kLanes * 8));
-                decode_sc<ELEM, 0>(tab, &ms, n0, make_uint4(0, 0, 0, 0), c0, c1, c2, p, qq);
+                decode_sc<ELEM, 0>(tab, n0, make_uint4(0, 0, 0, 0), c0, c1, c2, p, qq);
                 consume(2 * sp, p, qq);
                 if (2 * sp + 1 < nsc) {
                     const uint2 n1 = ldnt2((np + (uint64_t)(2 * sp + 1) * kLanes * 8));
-                    decode_sc<ELEM, 4>(tab, &ms, n1, make_uint4(0, 0, 0, 0), c0, c1, c2, p, qq);
+                    decode_sc<ELEM, 4>(tab, n1, make_uint4(0, 0, 0, 0), c0, c1, c2, p, qq);
                     consume(2 * sp + 1, p, qq);
                 }
             }
@@ -89,7 +88,7 @@ __global__ void __launch_bounds__(1024) k_layout2(BlockArgs a) {
                     rr = ldnt4((rp + (uint64_t)(sc + 1) * kLanes * 16));
                 }
                 uint32_t p[4], qq[4];
-                decode_sc<ELEM, 0>(tab, nullptr, nib, raw, 0u, 0u, 0u, p, qq);
+                decode_sc<ELEM, 0>(tab, nib, raw, 0u, 0u, 0u, p, qq);
                 consume(sc, p, qq);
             }
         }
@@ -122,20 +121,55 @@ __global__ void __launch_bounds__(1024) k_layout2(BlockArgs a) {
     if (MODE != kDequant) finish_rows<MODE>(a, part, rg0 * kRows12, ng * kRows12, f.CB, ELEM == kElemFp8 ? &fin : nullptr);
 }
 
-// BF16 token path: a workgroup owns G whole 16-row groups; each half-wave decodes super-chunks sc0 .. sc0 + NS - 1
-// of a block (SP = 16 / NS half-waves per block, so small matrices still fill the CUs; several blocks in turn when
-// the tile has more than fit), with its
-// nibble and raw loads four super-chunks ahead, the BF16 activations staged once per workgroup in LDS, and its lane's
-// exceptions whose super-chunk lies in its range (the fp32 path keeps k_layout2 and its fp32 products).  Partial row sums per (row, column block, part), summed in a fixed
-// order by the workgroup.  The fixed-width format needs no index to start inside a block.
-template <int MODE, bool XBF16, int NS>
+// A lane's exceptions, entries first, first + SP, ... (the SP half-waves of a block share them out: any of them can add any
+// entry, so each meets a quarter of the longest list of its lanes instead of reading all of it), N at a time.  The first
+// batch is in flight while the super-chunks decode; one dependent load per entry after them cost a memory round trip each.
+template <int ELEM, int SP>
+struct Exceptions {
+    static constexpr uint32_t N = (ELEM == kElemFp8 ? 4 : 2) * (SP == 4 ? 1 : 2), SIZE = ELEM == kElemFp8 ? 2 : 3;
+    typedef __attribute__((address_space(1))) const uint8_t byte_t;
+    typedef __attribute__((address_space(1), aligned(1))) const uint16_t any16_t;
+    byte_t *ep;
+    uint32_t cnt, next, v[N], top[N];
+    // a lane without entries reads bytes that are there (its block's header), never past `data`; the pointer is kept
+    // from the compiler, which would branch around the loads and wait inside the branch
+    __device__ __forceinline__ void init(const BlockArgs &a, uint32_t L, uint32_t n, uint32_t base, uint32_t first) {
+        cnt = n;
+        next = first;
+        const uint32_t incl = half_scan_incl(n, L);
+        uint64_t e = (uint64_t)(n ? a.data + base + (incl - n) * SIZE : a.hdr);
+        asm volatile("" : "+v"(e));
+        ep = (byte_t *)e;
+    }
+    __device__ __forceinline__ void request() {                  // past the last entry: the last again
+        const uint32_t last = max(cnt, 1u) - 1u;
+#pragma unroll
+        for (uint32_t k = 0; k < N; k++) {
+            byte_t *e = ep + min(next + k * SP, last) * SIZE;
+            v[k] = *(any16_t *)e;
+            if constexpr (ELEM != kElemFp8) top[k] = e[2];
+        }
+    }
+    __device__ __forceinline__ bool has(uint32_t k) const { return next + k * SP < cnt; }
+    __device__ __forceinline__ float value(uint32_t k) const {
+        if constexpr (ELEM == kElemFp8) return e4m3_to_f32((v[k] >> 8) & 0xFFu);
+        return __uint_as_float(top[k] << 24 | (v[k] & 0xFF00u) << 8);
+    }
+};
+
+// Token path: a workgroup owns G whole 16-row groups; each half-wave decodes super-chunks sc0 .. sc0 + NS - 1 of a block
+// (SP = 16 / NS half-waves per block, so small matrices still fill the CUs; several blocks in turn when the tile has more
+// than fit), with its nibble and raw loads four super-chunks ahead, the BF16 activations staged once per workgroup in
+// LDS, and its share of its lane's exceptions (the fp32 path keeps k_layout2 and its fp32
+// products).  Partial row sums per (row, column block, part), summed in a fixed order by the workgroup.  The fixed-width
+// format needs no index to start inside a block.
+template <int ELEM, int NS>
 __global__ void __launch_bounds__(1024) k_layout2s(BlockArgs a) {
     static_assert(NS == 4 || NS == 8 || NS == 16, "four, two or one half-wave per block");
-    static_assert(MODE == kToken && XBF16, "the BF16 token path");
     constexpr uint32_t SP = 16u / NS, R = 4;
+    constexpr bool FP8 = ELEM == kElemFp8;
     extern __shared__ uint32_t dyn[];
     const RankTab tab{a.lut[0], a.lut[1], a.lut[2], a.lut[3]};
-    constexpr uint32_t esz = 3u;
     const uint32_t tid = threadIdx.x, nth = blockDim.x, L = tid & 31, r = L >> 2, q = L & 3;
     const uint32_t hw = tid >> 5, H = nth >> 5;
     const Shape f(a.M, a.K, 2);
@@ -146,33 +180,61 @@ __global__ void __launch_bounds__(1024) k_layout2s(BlockArgs a) {
     const uint32_t rg0 = blockIdx.x * a.G;
     const uint32_t ng = min(a.G, f.groups() - rg0);
     const uint32_t nt = ng * f.CB;
-    for (uint32_t i = tid; i < n8; i += nth) xs[i] = ((const uint4 *)a.x)[i];
+    const RowFinish fin = row_finish_load<kToken, FP8>(a, rg0 * kRows12, ng * kRows12);
+    for (uint32_t i = tid; i < n8; i += nth) xs[i] = x8_settle<true>(x8_at<true>(a.x, 8u * i, f.K), 8u * i, f.K);
     __syncthreads();
     for (uint32_t it = hw; it < nt * SP; it += H) {
         const uint32_t t = it / SP, p = it - t * SP;
         const uint32_t g = t / f.CB, cb = t - g * f.CB, rb = rg0 + g, b = rb * f.CB + cb;
         const uint32_t nsc = ((cb == f.CB - 1 ? f.nl : 32u) + 1) / 2, slot0 = rb * f.spr + cb * 16;
         const uint32_t sc0 = p * NS, ns = sc0 < nsc ? min(NS, nsc - sc0) : 0u;
+        const uint32_t cnt = a.hdr[(uint64_t)b * kHdrBytes + L], base = a.bases[b];
         const uint8_t *np = a.low + ((uint64_t)(slot0 + sc0) * kLanes + L) * 8;
-        const uint8_t *rp = rplane + ((uint64_t)(slot0 + sc0) * kLanes + L) * 16;
-        // the ring: super-chunk i of the range in slot i % R; loads past the range re-read its last super-chunk
+        const uint8_t *rp = FP8 ? rplane + (((uint64_t)rb * f.spr2 + cb * 8 + sc0 / 2) * 3 * kLanes + L) * 4
+                                : rplane + ((uint64_t)(slot0 + sc0) * kLanes + L) * 16;
+        // the ring: super-chunk i of the range in slot i % R (fp8: the three words of chunks i, i + 1 in slot i % R, i
+        // even); loads past the range re-read its last super-chunk
         uint2 nr[R];
         uint4 rr[R];
         const uint32_t last = ns ? ns - 1u : 0u;
+        auto request = [&](uint32_t i) {
+            const uint32_t c = min(i, last);
+            nr[i % R] = ldnt2(np + (uint64_t)c * kLanes * 8);
+            if constexpr (FP8) {
+                if (i % 2u == 0u) {
+                    const uint8_t *pp = rp + (uint64_t)(c / 2u) * 3 * kLanes * 4;
+                    rr[i % R].x = ldnt1(pp);
+                    rr[i % R].y = ldnt1(pp + kLanes * 4);
+                    rr[i % R].z = ldnt1(pp + 2 * kLanes * 4);
+                }
+            } else {
+                rr[i % R] = ldnt4(rp + (uint64_t)c * kLanes * 16);
+            }
+        };
 #pragma unroll
-        for (uint32_t i = 0; i < R; i++) {
-            nr[i] = ldnt2(np + (uint64_t)min(i, last) * kLanes * 8);
-            rr[i] = ldnt4(rp + (uint64_t)min(i, last) * kLanes * 16);
-        }
+        for (uint32_t i = 0; i < R; i++) request(i);
+        Exceptions<ELEM, SP> X;
+        X.init(a, L, cnt, base, p);
+        X.request();
         float accA = 0.f, accB = 0.f;
 #pragma unroll
         for (uint32_t i = 0; i < NS; i++) {
             if (i >= ns) continue;                               // a last column block's missing super-chunks
             uint32_t pa[4], qa[4];
-            decode_sc<kElemBf16, 0>(tab, nullptr, nr[i % R], rr[i % R], 0u, 0u, 0u, pa, qa);
-            if (i + R < NS) {
-                nr[i % R] = ldnt2(np + (uint64_t)min(i + R, last) * kLanes * 8);
-                rr[i % R] = ldnt4(rp + (uint64_t)min(i + R, last) * kLanes * 16);
+            if constexpr (FP8) {
+                const uint4 c = rr[(i % R) & ~1u];
+                if (i % 2u) decode_sc<ELEM, 4>(tab, nr[i % R], c, c.x, c.y, c.z, pa, qa);
+                else decode_sc<ELEM, 0>(tab, nr[i % R], c, c.x, c.y, c.z, pa, qa);
+            } else {
+                decode_sc<ELEM, 0>(tab, nr[i % R], rr[i % R], 0u, 0u, 0u, pa, qa);
+            }
+            if constexpr (FP8) {
+                if (i % 2u && i + R - 1u < NS) {
+                    request(i + R - 1u);
+                    request(i + R);
+                }
+            } else {
+                if (i + R < NS) request(i + R);
             }
             const uint4 xv = xs[(cb * kCols + (sc0 + i) * 32u + 8u * q) >> 3];
 #pragma unroll
@@ -182,17 +244,19 @@ __global__ void __launch_bounds__(1024) k_layout2s(BlockArgs a) {
             }
             asm volatile("" : "+v"(accA), "+v"(accB));
         }
-        // exceptions of this lane whose super-chunk is in the range (planes decoded to +-0, the entries carry the value)
-        uint32_t cnt;
-        const uint8_t *ep = exc_start(a, b, L, esz, cnt);
-        for (uint32_t k = 0; k < cnt; k++, ep += esz) {
-            const uint32_t i = ep[0], j = i & 15, sc = i >> 4;
-            if (sc - sc0 >= ns) continue;
-            const uint32_t col = cb * kCols + sc * 32 + frag_col(L, j), upper = (j >> 1) & 1u;
-            const float w = exc_value<kElemBf16>(ep);
-            const float xv = __uint_as_float((uint32_t)((const uint16_t *)xs)[col] << 16);
-            if (upper) accB = fmaf(w, xv, accB);
-            else accA = fmaf(w, xv, accA);
+        // this half-wave's share of the lane's exceptions (planes decoded to +-0, the entries carry the value)
+        while (__any(X.has(0u))) {
+#pragma unroll
+            for (uint32_t k = 0; k < X.N; k++) {
+                if (!X.has(k)) continue;
+                const uint32_t i = X.v[k] & 0xFFu, j = i & 15;
+                const uint32_t col = cb * kCols + (i >> 4) * 32 + frag_col(L, j), upper = (j >> 1) & 1u;
+                const float xv = __uint_as_float((uint32_t)((const uint16_t *)xs)[col] << 16), w = X.value(k);
+                if (upper) accB = fmaf(w, xv, accB);
+                else accA = fmaf(w, xv, accA);
+            }
+            X.next += X.N * SP;
+            if (__any(X.has(0u))) X.request();
         }
         accA += xor_f<1>(accA); accA += xor_f<2>(accA);
         accB += xor_f<1>(accB); accB += xor_f<2>(accB);
@@ -202,14 +266,12 @@ __global__ void __launch_bounds__(1024) k_layout2s(BlockArgs a) {
             part[pi + 8u * f.CB * SP] = accB;
         }
     }
-    finish_rows<MODE>(a, part, rg0 * kRows12, ng * kRows12, f.CB * SP);
+    finish_rows<kToken>(a, part, rg0 * kRows12, ng * kRows12, f.CB * SP, FP8 ? &fin : nullptr);
 }
 
 // Row gather: one half-wave per requested row; the row's lanes store their columns, then patch their exceptions.
 template <int ELEM>
 __global__ void __launch_bounds__(256) k_gather2(GatherArgs a) {
-    __shared__ MantLds ms;
-    if (ELEM == kElemFp8) stage_mant(ms);
     const RankTab tab{a.lut[0], a.lut[1], a.lut[2], a.lut[3]};
     constexpr uint32_t esz = ELEM == kElemFp8 ? 2u : 3u;
     const uint32_t L = threadIdx.x & 31, r = L >> 2, q = L & 3;
@@ -253,10 +315,10 @@ __global__ void __launch_bounds__(256) k_gather2(GatherArgs a) {
         if (i > last) break;
         uint32_t pv[4], qv[4];
         if constexpr (ELEM == kElemFp8) {
-            if (i & 1u) decode_sc<ELEM, 4>(tab, &ms, nib[i], make_uint4(0, 0, 0, 0), c[i / 2][0], c[i / 2][1], c[i / 2][2], pv, qv);
-            else decode_sc<ELEM, 0>(tab, &ms, nib[i], make_uint4(0, 0, 0, 0), c[i / 2][0], c[i / 2][1], c[i / 2][2], pv, qv);
+            if (i & 1u) decode_sc<ELEM, 4>(tab, nib[i], make_uint4(0, 0, 0, 0), c[i / 2][0], c[i / 2][1], c[i / 2][2], pv, qv);
+            else decode_sc<ELEM, 0>(tab, nib[i], make_uint4(0, 0, 0, 0), c[i / 2][0], c[i / 2][1], c[i / 2][2], pv, qv);
         } else {
-            decode_sc<ELEM, 0>(tab, nullptr, nib[i], raw[i], 0u, 0u, 0u, pv, qv);
+            decode_sc<ELEM, 0>(tab, nib[i], raw[i], 0u, 0u, 0u, pv, qv);
         }
         const uint32_t kc = cb * kCols + (sc0 + i) * 32 + 8 * q;
         if (mine && kc < f.K16) {
@@ -281,11 +343,11 @@ __global__ void __launch_bounds__(256) k_gather2(GatherArgs a) {
 
 template <int ELEM, int MODE, bool XBF16>
 static int launch_fixed_t(const LaunchPlan &p, const BlockArgs &a, hipStream_t st) {
-    if constexpr (ELEM == kElemBf16 && MODE == kToken && XBF16) {
+    if constexpr (MODE == kToken && XBF16) {
         if (p.split) {
-            if (p.split == 4) hipLaunchKernelGGL((k_layout2s<MODE, XBF16, 4>), dim3(p.grid), dim3(p.threads), p.lds, st, a);
-            else if (p.split == 2) hipLaunchKernelGGL((k_layout2s<MODE, XBF16, 8>), dim3(p.grid), dim3(p.threads), p.lds, st, a);
-            else hipLaunchKernelGGL((k_layout2s<MODE, XBF16, 16>), dim3(p.grid), dim3(p.threads), p.lds, st, a);
+            if (p.split == 4) hipLaunchKernelGGL((k_layout2s<ELEM, 4>), dim3(p.grid), dim3(p.threads), p.lds, st, a);
+            else if (p.split == 2) hipLaunchKernelGGL((k_layout2s<ELEM, 8>), dim3(p.grid), dim3(p.threads), p.lds, st, a);
+            else hipLaunchKernelGGL((k_layout2s<ELEM, 16>), dim3(p.grid), dim3(p.threads), p.lds, st, a);
             return (int)hipGetLastError();
         }
     }

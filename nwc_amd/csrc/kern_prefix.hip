@@ -38,12 +38,14 @@ __device__ __forceinline__ uint4 raw_row0(const uint8_t *__restrict__ low, const
     return ldnt4(low + (r * f.K16 + c));
 }
 
+// K: a.K, for BF16 activations that end inside the lane's 16 columns (settle_x16 puts those in place once they have
+// arrived); 0 where x is zero-extended.  The address is clamped, not branched on: a load inside a branch would be waited for.
 template <bool XBF16>
-__device__ __forceinline__ void load_x16(XRegs<XBF16> &x, const void *xp, uint32_t col0, bool col_ok) {
+__device__ __forceinline__ void load_x16(XRegs<XBF16> &x, const void *xp, uint32_t col0, bool col_ok, uint32_t K = 0) {
     const uint32_t c = col_ok ? col0 : 0u;
     if constexpr (XBF16) {
-        const uint4 *p = (const uint4 *)((const uint16_t *)xp + c);
-        const uint4 v0 = p[0], v1 = p[1];
+        const uint16_t *p = (const uint16_t *)xp + (K >= 16u ? min(c, K - 16u) : c);
+        const uint4 v0 = ld_any4(p), v1 = ld_any4(p + 8);
         x.b[0] = v0.x; x.b[1] = v0.y; x.b[2] = v0.z; x.b[3] = v0.w; x.b[4] = v1.x; x.b[5] = v1.y; x.b[6] = v1.z; x.b[7] = v1.w;
     } else {
 #pragma unroll
@@ -51,6 +53,12 @@ __device__ __forceinline__ void load_x16(XRegs<XBF16> &x, const void *xp, uint32
             const float4 v = ((const float4 *)((const float *)xp + c))[i];
             x.f[4 * i] = v.x; x.f[4 * i + 1] = v.y; x.f[4 * i + 2] = v.z; x.f[4 * i + 3] = v.w;
         }
+    }
+}
+template <bool XBF16>
+__device__ __forceinline__ void settle_x16(XRegs<XBF16> &x, uint32_t col0, bool col_ok, uint32_t K) {
+    if constexpr (XBF16) {
+        if ((K & 15u) != 0u && K >= 16u) shift_down<8>(x.b, col_ok && col0 + 16u > K ? col0 + 16u - K : 0u);
     }
 }
 
@@ -225,7 +233,7 @@ __device__ __forceinline__ float rows0_ring(const LutLds &s, const uint32_t *wor
     for (int r = 0; r < (int)kRows0; r++) {
         if (r == 4) {
             bulk_issue(Bk, a.data, Rn, tid, nth);
-            if (MODE == kToken || MODE == kF32) load_x16<XBF16>(xn, a.x, nx.col0, nx.col_ok);
+            if (MODE == kToken || MODE == kF32) load_x16<XBF16>(xn, a.x, nx.col0, nx.col_ok, f.K);
         }
         if (MODE == kRowIndex && r > 0 && (r & 1) == 0 && valid)
             ((uint16_t *)a.out)[((uint64_t)c.b * kRowIndexSplits + (r >> 1) - 1) * kLanes + L] = (uint16_t)S.position(words);
@@ -349,7 +357,7 @@ __device__ __forceinline__ void layout0_body(BlockArgs a, uint32_t nth, uint32_t
     Bulk Bk;
     bulk_issue(Bk, a.data, R, tid, nth);
     XRegs<XBF16> x;
-    if (ROWS) load_x16<XBF16>(x, a.x, c.col0, c.col_ok);
+    if (ROWS) load_x16<XBF16>(x, a.x, c.col0, c.col_ok, f.K);
     // the finish's scale and bias after the streams: the preloaded kernels read those pointers from their argument
     // struct, and the wait for that read must not hold back the requests above
     const RowFinish fin = PART ? row_finish_load<MODE>(a, rg0 * kRows0 + r0, NR, flags)
@@ -372,6 +380,7 @@ __device__ __forceinline__ void layout0_body(BlockArgs a, uint32_t nth, uint32_t
         for (int r = 0; r < (NR < RING ? NR : RING); r++)
             raw[r] = MODE == kRowIndex ? make_uint4(0u, 0u, 0u, 0u) : raw_row<ELEM>(a.low, f, c, r);
         if (t < nt) {
+            if (ROWS) settle_x16<XBF16>(x, c.col0, c.col_ok, f.K);
             const uint32_t start = c.col_ok ? half_scan_incl(n, L) - n : 0u;
             float v;
             if (fits) v = rowsN<ELEM, MODE, XBF16, NR>(s, cur + ((base - R.lo16) >> 2) + start, P0, a, f, x, raw, c, r0, L);
@@ -393,6 +402,7 @@ __device__ __forceinline__ void layout0_body(BlockArgs a, uint32_t nth, uint32_t
         Q.finish(s, a, nth);
         if (R.n16 * 4u <= cap) bulk_commit(Bk, cur, R, tid, nth);
         __syncthreads();
+        if (ROWS) settle_x16<XBF16>(x, c.col0, c.col_ok, f.K);
         const uint32_t rounds = (nt + H - 1u) / H;
         uint32_t start = c.col_ok ? half_scan_incl(n, L) - n : 0u;
         for (uint32_t k = 0;; k++) {
@@ -408,7 +418,7 @@ __device__ __forceinline__ void layout0_body(BlockArgs a, uint32_t nth, uint32_t
                                                   Rn, xn, tid, nth, L);
             } else {
                 bulk_issue(Bk, a.data, Rn, tid, nth);
-                if (ROWS) load_x16<XBF16>(xn, a.x, cn.col0, cn.col_ok);
+                if (ROWS) load_x16<XBF16>(xn, a.x, cn.col0, cn.col_ok, f.K);
                 v = rows0_global<ELEM, MODE, XBF16>(s, (const uint32_t *)(a.data + base) + start, a, f, x, c, valid, L);
 #pragma unroll
                 for (int r = 0; r < 4; r++) ring[r] = MODE == kRowIndex ? make_uint4(0u, 0u, 0u, 0u) : raw_row<ELEM>(a.low, f, cn, r);
@@ -422,7 +432,10 @@ __device__ __forceinline__ void layout0_body(BlockArgs a, uint32_t nth, uint32_t
             base = base_n;
             R = Rn;
             Rn = Rnn;
-            if (ROWS) x = xn;
+            if (ROWS) {
+                x = xn;
+                settle_x16<XBF16>(x, cn.col0, cn.col_ok, f.K);
+            }
             c = cn;
             cn = cnn;
             n_n = n_nn;
@@ -546,7 +559,8 @@ __device__ __forceinline__ float2 rows1(const LutLds &s, P words, const BlockArg
         uint4 xv = make_uint4(0, 0, 0, 0);
         float xf[8];
         if (MODE != kDequant) {
-            if (XBF16) xv = *(const uint4 *)((const uint16_t *)a.x + kc);
+            if (XBF16) xv = kc + 8u <= f.K || f.K < 16u ? *(const uint4 *)((const uint16_t *)a.x + kc)
+                                                        : x8_tail((const uint16_t *)a.x, kc, f.K);
             else {
                 const float4 x0 = ((const float4 *)((const float *)a.x + kc))[0], x1 = ((const float4 *)((const float *)a.x + kc))[1];
                 xf[0] = x0.x; xf[1] = x0.y; xf[2] = x0.z; xf[3] = x0.w; xf[4] = x1.x; xf[5] = x1.y; xf[6] = x1.z; xf[7] = x1.w;
@@ -627,15 +641,6 @@ __global__ void __launch_bounds__(1024) k_layout1(BlockArgs a) {
 // (SP = 16 / NS half-waves per block; with SP > 1 the row index gives each lane's bit position at super-chunk
 // 4, 8, 12).  Raw super-chunks go through a ring of two registers (chunk s + 2 is requested when chunk s is done).  Partial row sums are kept per (row, column block, part) and summed in a fixed
 // order by the workgroup.
-// Eight activations from kc as BF16 pairs (fp32 x: rounded to BF16, as the reference's fp32 path does for layouts
-// 1/2).  x holds K32 values, so every coded super-chunk is in bounds.
-template <bool XBF16>
-__device__ __forceinline__ uint4 x8_at(const void *x, uint32_t kc) {
-    if constexpr (XBF16) return *(const uint4 *)((const uint16_t *)x + kc);
-    const float4 a = ((const float4 *)((const float *)x + kc))[0], b = ((const float4 *)((const float *)x + kc))[1];
-    return make_uint4(f32_to_bf16_rne(a.x) | f32_to_bf16_rne(a.y) << 16, f32_to_bf16_rne(a.z) | f32_to_bf16_rne(a.w) << 16,
-                      f32_to_bf16_rne(b.x) | f32_to_bf16_rne(b.y) << 16, f32_to_bf16_rne(b.z) | f32_to_bf16_rne(b.w) << 16);
-}
 // The activations are staged once per workgroup as BF16 in LDS, so their per-super-chunk reads are LDS reads: a global
 // load there would be waited for in issue order together with the raw chunks requested before it.
 // In three parts, as the decode table is staged: the first two chunks per thread are requested with the prologue's
@@ -643,18 +648,18 @@ __device__ __forceinline__ uint4 x8_at(const void *x, uint32_t kc) {
 // them, the streams included); x_finish copies the rest (fewer than n8 / 2 threads).
 template <bool XBF16> struct XStage { uint4 v0, v1; };
 template <bool XBF16>
-__device__ __forceinline__ void x_issue(XStage<XBF16> &X, const void *x, uint32_t n8, uint32_t tid, uint32_t nth) {
-    X.v0 = x8_at<XBF16>(x, 8u * min(tid, n8 - 1u));
-    X.v1 = x8_at<XBF16>(x, 8u * min(tid + nth, n8 - 1u));
+__device__ __forceinline__ void x_issue(XStage<XBF16> &X, const void *x, uint32_t K, uint32_t n8, uint32_t tid, uint32_t nth) {
+    X.v0 = x8_at<XBF16>(x, 8u * min(tid, n8 - 1u), K);
+    X.v1 = x8_at<XBF16>(x, 8u * min(tid + nth, n8 - 1u), K);
 }
 template <bool XBF16>
-__device__ __forceinline__ void x_commit(const XStage<XBF16> &X, uint4 *xs, uint32_t n8, uint32_t tid, uint32_t nth) {
-    if (tid < n8) xs[tid] = X.v0;
-    if (tid + nth < n8) xs[tid + nth] = X.v1;
+__device__ __forceinline__ void x_commit(const XStage<XBF16> &X, uint4 *xs, uint32_t K, uint32_t n8, uint32_t tid, uint32_t nth) {
+    if (tid < n8) xs[tid] = x8_settle<XBF16>(X.v0, 8u * tid, K);
+    if (tid + nth < n8) xs[tid + nth] = x8_settle<XBF16>(X.v1, 8u * (tid + nth), K);
 }
 template <bool XBF16>
-__device__ __forceinline__ void x_finish(uint4 *xs, const void *x, uint32_t n8, uint32_t tid, uint32_t nth) {
-    for (uint32_t i = tid + 2u * nth; i < n8; i += nth) xs[i] = x8_at<XBF16>(x, 8u * i);
+__device__ __forceinline__ void x_finish(uint4 *xs, const void *x, uint32_t K, uint32_t n8, uint32_t tid, uint32_t nth) {
+    for (uint32_t i = tid + 2u * nth; i < n8; i += nth) xs[i] = x8_settle<XBF16>(x8_at<XBF16>(x, 8u * i, K), 8u * i, K);
 }
 
 // Raw super-chunks in flight per half-wave in the single-round kernel: two, as for layout 0's rows.
@@ -816,7 +821,7 @@ __device__ __forceinline__ void layout1s_body(BlockArgs a, uint32_t nth, uint32_
     Bulk Bk;
     bulk_issue(Bk, a.data, R, tid, nth);
     XStage<XBF16> X;
-    if (ROWS) x_issue<XBF16>(X, a.x, n8, tid, nth);
+    if (ROWS) x_issue<XBF16>(X, a.x, f.K, n8, tid, nth);
     // fp8: the finish's row scale after the streams (the preloaded kernel reads its pointer from the argument struct,
     // and the wait for that read must not hold back the requests above)
     const RowFinish fin = row_finish_load<MODE, ELEM == kElemFp8>(a, rg0 * kRows12, ng * kRows12, flags);
@@ -825,8 +830,8 @@ __device__ __forceinline__ void layout1s_body(BlockArgs a, uint32_t nth, uint32_
     const uint32_t P0 = SP == 1 ? 0u : part_start(a, c.b, sc0 / 4u, L);
     Q.commit(s, nth);
     if (ROWS) {
-        x_commit<XBF16>(X, xs, n8, tid, nth);
-        x_finish<XBF16>(xs, a.x, n8, tid, nth);
+        x_commit<XBF16>(X, xs, f.K, n8, tid, nth);
+        x_finish<XBF16>(xs, a.x, f.K, n8, tid, nth);
     }
     Q.finish(s, a, nth);
     // the copy moves four 16-byte chunks per thread (512 words per half-wave); a larger region (one half-wave per
@@ -924,9 +929,9 @@ __device__ __forceinline__ void layout1m_body(BlockArgs a, uint32_t nth, uint32_
     // measured faster here than k_layout1s's: 2560x9728 15.8 us against 16.6-17.0, the later ones leaving the
     // compiler a register choice that waits inside the item loop)
     XStage<true> X;
-    x_issue<true>(X, a.x, n8, tid, nth);
-    x_commit<true>(X, xs, n8, tid, nth);
-    x_finish<true>(xs, a.x, n8, tid, nth);
+    x_issue<true>(X, a.x, f.K, n8, tid, nth);
+    x_commit<true>(X, xs, f.K, n8, tid, nth);
+    x_finish<true>(xs, a.x, f.K, n8, tid, nth);
     Q.commit(s, nth);
     Q.finish(s, a, nth);
     uint4 ring[4];

@@ -455,8 +455,6 @@ struct ExcCursor {                                               // a lane's nex
 template <int ELEM, int NT>
 __global__ void __launch_bounds__(kTokensMaxWaves * 64) k_tokens2(TokensArgs p) {
     const BlockArgs &a = p.a;
-    __shared__ uint32_t mant[ELEM == kElemFp8 ? kLutWords : 4];
-    MantLds *ms = (MantLds *)mant;
     extern __shared__ __attribute__((aligned(16))) uint32_t dyn[];
     const uint32_t tid = threadIdx.x, lane = tid & 63u, wv = tid >> 6, L = tid & 31u, h = lane >> 5;
     const uint32_t i16 = lane & 15u, c4 = lane >> 4;
@@ -488,7 +486,6 @@ __global__ void __launch_bounds__(kTokensMaxWaves * 64) k_tokens2(TokensArgs p) 
     for (uint32_t i = 0; i < 8; i++) request(w.unit, i);
     uint32_t *xs = dyn, *patch = dyn + NT * 16u * kTokensXRow + wv * kTokensPatchWords;
     S.commit(xs, p, w.cb);
-    if constexpr (ELEM == kElemFp8) stage_mant(*ms);
     __syncthreads();
     const uint32_t r = L >> 2, q = L & 3u;
     uint32_t *wa = patch + 256u * h + 16u * r + 4u * ((q ^ (r >> 2)) & 3u);
@@ -509,10 +506,10 @@ __global__ void __launch_bounds__(kTokensMaxWaves * 64) k_tokens2(TokensArgs p) 
                 uint32_t pa[4], pb[4];
                 if constexpr (ELEM == kElemFp8) {
                     const uint4 c = raw[i & ~1u];
-                    if (i & 1u) decode_sc<ELEM, 4>(tab, ms, nib[i], c, c.x, c.y, c.z, pa, pb);
-                    else decode_sc<ELEM, 0>(tab, ms, nib[i], c, c.x, c.y, c.z, pa, pb);
+                    if (i & 1u) decode_sc<ELEM, 4>(tab, nib[i], c, c.x, c.y, c.z, pa, pb);
+                    else decode_sc<ELEM, 0>(tab, nib[i], c, c.x, c.y, c.z, pa, pb);
                 } else {
-                    decode_sc<ELEM, 0>(tab, nullptr, nib[i], raw[i], 0u, 0u, 0u, pa, pb);
+                    decode_sc<ELEM, 0>(tab, nib[i], raw[i], 0u, 0u, 0u, pa, pb);
                 }
                 *(uint4 *)wa = make_uint4(pa[0], pa[1], pa[2], pa[3]);
                 *(uint4 *)wb = make_uint4(pb[0], pb[1], pb[2], pb[3]);

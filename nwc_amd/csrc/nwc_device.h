@@ -37,6 +37,60 @@ __device__ __forceinline__ uint2 ldnt2(const void *p) {
 }
 __device__ __forceinline__ uint32_t ldnt1(const void *p) { return __builtin_nontemporal_load((const uint32_t *)p); }
 
+// ---- BF16 activations that end inside a 16-byte piece (K not a multiple of 8, 16 or 32) ----
+// x holds K values and nothing past them is read (K >= 16): a piece that would cross the end is read K - 8 (K - 16)
+// values in, at any 2-byte boundary, and moved down by the values it starts too early, zeros coming in at the top.
+// Without a tail neither happens.  This saves the callers the two launches of a padded copy (10 us of host time).
+typedef __attribute__((ext_vector_type(4), aligned(2))) uint32_t u32x4_any;
+__device__ __forceinline__ uint4 ld_any4(const uint16_t *p) {
+    const u32x4_t v = *(const u32x4_any *)p;
+    return make_uint4(v.x, v.y, v.z, v.w);
+}
+// N words moved down by `n` 16-bit values (0 <= n < 2 N; n >= 2 N: all zero for N = 4)
+template <int N>
+__device__ __forceinline__ void shift_down(uint32_t (&w)[N], uint32_t n) {
+#pragma unroll
+    for (int i = 0; i < N; i++) {
+        const uint32_t up = i + 1 < N ? w[i + 1] : 0u;
+        w[i] = n & 1u ? (w[i] >> 16) | (up << 16) : w[i];
+    }
+#pragma unroll
+    for (int b = 1; b < N; b *= 2) {
+#pragma unroll
+        for (int i = 0; i < N; i++) {
+            const uint32_t up = i + b < N ? w[i + b] : 0u;
+            w[i] = n & (2u * b) ? up : w[i];
+        }
+    }
+}
+// the eight activations from column kc, zero past K (any kc)
+__device__ __forceinline__ uint4 x8_tail(const uint16_t *x, uint32_t kc, uint32_t K) {
+    const uint32_t c = min(kc, K - 8u);
+    const uint4 v = ld_any4(x + c);
+    uint32_t w[4] = {v.x, v.y, v.z, v.w};
+    shift_down<4>(w, kc - c);
+    const uint32_t keep = kc < K ? ~0u : 0u;
+    return make_uint4(w[0] & keep, w[1] & keep, w[2] & keep, w[3] & keep);
+}
+
+// Eight activations from kc as BF16 pairs (fp32 x: rounded to BF16, as the reference's fp32 path does for layouts
+// 1/2).  fp32 x holds K32 values, so every coded super-chunk is in bounds; BF16 x ends at K (x8_settle).
+template <bool XBF16>
+__device__ __forceinline__ uint4 x8_at(const void *x, uint32_t kc, uint32_t K) {
+    if constexpr (XBF16) return ld_any4((const uint16_t *)x + (K >= 16u ? min(kc, K - 8u) : kc));
+    const float4 a = ((const float4 *)((const float *)x + kc))[0], b = ((const float4 *)((const float *)x + kc))[1];
+    return make_uint4(f32_to_bf16_rne(a.x) | f32_to_bf16_rne(a.y) << 16, f32_to_bf16_rne(a.z) | f32_to_bf16_rne(a.w) << 16,
+                      f32_to_bf16_rne(b.x) | f32_to_bf16_rne(b.y) << 16, f32_to_bf16_rne(b.z) | f32_to_bf16_rne(b.w) << 16);
+}
+// x8_at's piece in its place once it has arrived: moved down where it was read early, zero past K
+template <bool XBF16>
+__device__ __forceinline__ uint4 x8_settle(const uint4 &v, uint32_t kc, uint32_t K) {
+    if (!XBF16 || (K & 31u) == 0u || K < 16u) return v;
+    uint32_t w[4] = {v.x, v.y, v.z, v.w};
+    shift_down<4>(w, kc - min(kc, K - 8u));
+    const uint32_t keep = kc < K ? ~0u : 0u;
+    return make_uint4(w[0] & keep, w[1] & keep, w[2] & keep, w[3] & keep);
+}
 // Byte selectors for v_perm_b32(e, raw, sel): bytes 0-3 of `raw`, 4-7 of `e` (e byte 1/2 = exponent bytes of the
 // pair), 0x0C = zero byte.  A BF16 pair [raw_j | e1][raw_j+1 | e2] (j = 0 or 2 inside the raw word):
 constexpr uint32_t kSelPair0 = 0x06010500u;   // weights 0,1 of a raw word

@@ -27,11 +27,11 @@ __device__ __forceinline__ void ranks8(const RankTab &t, uint32_t nw, uint32_t &
 constexpr uint32_t kSelLoHi01 = 0x05010400u;
 constexpr uint32_t kSelLoHi23 = 0x07030602u;
 
-// bits 12G .. 12G+11 of the 96-bit little-endian integer w2:w1:w0 (G a compile-time constant after unrolling)
+// bits 12G .. 12G+11 (and what follows them above) of the 96-bit little-endian integer w2:w1:w0 (G a compile-time constant after unrolling)
 __device__ __forceinline__ uint32_t bits12(uint32_t w0, uint32_t w1, uint32_t w2, int G) {
     const int bit = 12 * G, k = bit >> 5, sh = bit & 31;
     const uint32_t lo = k == 0 ? w0 : k == 1 ? w1 : w2, hi = k == 0 ? w1 : k == 1 ? w2 : 0u;
-    return __builtin_amdgcn_alignbit(hi, lo, (uint32_t)sh) & 0xFFFu;
+    return __builtin_amdgcn_alignbit(hi, lo, (uint32_t)sh);
 }
 
 __device__ __forceinline__ float e4m3_to_f32(uint32_t b) {
@@ -46,17 +46,16 @@ __device__ __forceinline__ float exc_value(const uint8_t *e) {
     return __uint_as_float(((uint32_t)e[1] | ((uint32_t)e[2] << 8)) << 16);
 }
 
-// fp8: 12-bit index (four 3-bit fields) -> the four fields, each shifted into bits 4..6 of its byte
-struct MantLds { uint32_t m[kLutWords]; };
-__device__ __forceinline__ void stage_mant(MantLds &s) {
-    for (uint32_t i = threadIdx.x; i < kLutWords; i += blockDim.x)
-        s.m[i] = ((i & 7u) << 4) | (((i >> 3) & 7u) << 12) | (((i >> 6) & 7u) << 20) | (((i >> 9) & 7u) << 28);
-    __syncthreads();
+// fp8: the four 3-bit fields of a 12-bit value, each in bits 4..6 of its byte (six operations; a 4096-entry LDS table
+// instead cost a random read per four weights and its staging: k_layout2s, 6144 x 2560 fp8, 17.5 us with it)
+__device__ __forceinline__ uint32_t mant4(uint32_t v) {
+    const uint32_t y = (v & 0x3Fu) | ((v << 10) & 0x3F0000u);
+    return ((y << 4) | (y << 9)) & 0x70707070u;
 }
 
 // Decodes one super-chunk of a lane: p[k] = BF16 pair of row r (positions 4k, 4k+1), q[k] = pair of row r+8.
 template <int ELEM, int G0>
-__device__ __forceinline__ void decode_sc(const RankTab &t, const MantLds *ms, uint2 nib, uint4 raw, uint32_t c0, uint32_t c1, uint32_t c2,
+__device__ __forceinline__ void decode_sc(const RankTab &t, uint2 nib, uint4 raw, uint32_t c0, uint32_t c1, uint32_t c2,
                                           uint32_t p[4], uint32_t q[4]) {
 #pragma unroll
     for (int h = 0; h < 2; h++) {
@@ -64,8 +63,8 @@ __device__ __forceinline__ void decode_sc(const RankTab &t, const MantLds *ms, u
         ranks8(t, h ? nib.y : nib.x, h03, h47, l03, l47, ELEM == kElemFp8);
         uint32_t r0, r1;                                          // low bytes of positions 8h+0..3 and 8h+4..7
         if (ELEM == kElemFp8) {
-            r0 = ms->m[bits12(c0, c1, c2, G0 + 2 * h)] | l03;
-            r1 = ms->m[bits12(c0, c1, c2, G0 + 2 * h + 1)] | l47;
+            r0 = mant4(bits12(c0, c1, c2, G0 + 2 * h)) | l03;
+            r1 = mant4(bits12(c0, c1, c2, G0 + 2 * h + 1)) | l47;
         } else {
             r0 = h ? raw.z : raw.x;
             r1 = h ? raw.w : raw.y;

@@ -521,7 +521,9 @@ class NWCWeight:
         y = torch.empty(self.out_features, dtype=torch.bfloat16, device=x.device)
         if x.dtype == torch.bfloat16 or self.layout:
             # BF16 activations (layouts 1/2 always take them): the extended entry point with the derived structures
-            xin = self._padded(x.to(torch.bfloat16))
+            xin = x.to(torch.bfloat16)
+            if self.in_features < 16 or not xin.is_contiguous() or xin.data_ptr() % 16:
+                xin = self._padded(xin)                # (otherwise the kernels read the in_features values and no more)
             call("nwc_linear_xbf16", stream(), *self._streams(), ptr(self.row_index()), ptr(self.seq_table()),
                  ptr(xin), ptr(bias), ptr(self.scale), ptr(y), self.n, self.in_features, self.code)
         else:
