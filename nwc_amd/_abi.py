@@ -44,6 +44,12 @@ SIGNATURES = {
 # entry points for this package alone (nwc_amd/csrc/nwc_private.h), not part of the C ABI
 PRIVATE = {
     "nwc_tokens": ("i", "pppppppppIppppQQIiI"),
+    "nwc_encode_supported": ("i", "QIi"),
+    "nwc_encode_hist": ("i", "ppQip"),
+    "nwc_encode_rank": ("i", "pipp"),
+    "nwc_encode_sizes": ("i", "ppQIipppp"),
+    "nwc_encode_write": ("i", "ppQIippppp"),
+    "nwc_copy_spans": ("i", "ppppppI"),
 }
 
 

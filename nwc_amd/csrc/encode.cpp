@@ -7,6 +7,7 @@
 // writes every block straight to its final offset.  No temporary copy of the matrix is made.
 #include "nwc_format.h"
 #include "nwc_ops.h"
+#include "nwc_private.h"
 
 #include <algorithm>
 #include <array>
@@ -109,6 +110,25 @@ void rank_symbols(const uint64_t hist[128], int nsym, int ord[128]) {
             if (hist[ord[b]] > hist[ord[a]]) std::swap(ord[a], ord[b]);
 }
 
+// The symbols' ranks (layout 2: at most 7, an exception) and the psym buffer from the symbol counts.
+void rank_and_psym(const uint64_t hist[128], int t, int lay, uint8_t rank[128], uint16_t *psym) {
+    const int nsym = t == kElemFp8 ? (lay == 2 ? 20 : 10) : 128;
+    int ord[128];
+    rank_symbols(hist, nsym, ord);
+    for (int r = 0; r < 128; r++) rank[ord[r]] = (uint8_t)(lay == 2 ? std::min(r, 7) : r);
+    for (uint32_t i = 0; i < kNpsym; i++) psym[i] = 0;
+    if (lay == 2) {
+        const auto &T = fp8_tables();
+        for (int r = 0; r < 7; r++) {
+            psym[r] = (uint16_t)(t == kElemFp8 ? T.hb2[ord[r]] : ord[r]);
+            psym[8 + r] = (uint16_t)(t == kElemFp8 ? T.lb2[ord[r]] : 0);
+        }
+        return;
+    }
+    static const uint8_t kFp8Byte3[10] = {60, 61, 62, 63, 64, 65, 66, 67, 59, 0};
+    for (int i = 0; i < 16; i++) psym[i] = (uint16_t)(t == kElemFp8 ? (i < 10 ? kFp8Byte3[ord[i]] : 0) : ord[i]);
+}
+
 // MSB-first code words, little-endian 32-bit words in memory.
 struct WordSink {
     uint8_t *dst; uint64_t acc = 0; int n = 0; uint32_t words = 0;
@@ -133,7 +153,6 @@ inline LanePos lane_pos(int lay, uint32_t rb, uint32_t cb, uint32_t L, uint32_t 
 // ---- layouts 0 and 1 -------------------------------------------------------------------------------------
 int64_t encode_prefix(const Splitter &S, const Shape &f, uint64_t K, int t, int lay, uint16_t *psym, uint32_t *bases,
                       uint8_t *hdr, uint8_t *data, uint64_t cap, uint8_t *low) {
-    const int nsym = t == kElemFp8 ? 10 : 128;
     const uint32_t maxr = t == kElemFp8 ? kMaxRankFp8 : kMaxRankBf16;
     const uint64_t n = (uint64_t)f.M * K;
 
@@ -147,13 +166,8 @@ int64_t encode_prefix(const Splitter &S, const Shape &f, uint64_t K, int t, int 
     });
     uint64_t hist[128] = {0};
     for (int s = 0; s < slot; s++) for (int k = 0; k < 128; k++) hist[k] += part[s][k];
-    int ord[128];
-    rank_symbols(hist, nsym, ord);
     uint8_t rank[128];
-    for (int r = 0; r < 128; r++) rank[ord[r]] = (uint8_t)r;
-    static const uint8_t kFp8Byte3[10] = {60, 61, 62, 63, 64, 65, 66, 67, 59, 0};
-    for (uint32_t i = 0; i < kNpsym; i++) psym[i] = 0;
-    for (int i = 0; i < 16; i++) psym[i] = (uint16_t)(t == kElemFp8 ? (i < 10 ? kFp8Byte3[ord[i]] : 0) : ord[i]);
+    rank_and_psym(hist, t, lay, rank, psym);
 
     // code length of each high byte (sign | symbol)
     uint8_t clen[256];
@@ -252,10 +266,8 @@ int64_t encode_prefix(const Splitter &S, const Shape &f, uint64_t K, int t, int 
 // ---- layout 2 --------------------------------------------------------------------------------------------
 int64_t encode_fixed(const Splitter &S, const void *wv, const Shape &f, uint64_t K, int t, uint16_t *psym,
                      uint32_t *bases, uint8_t *hdr, uint8_t *data, uint64_t cap, uint8_t *low) {
-    const int nsym = t == kElemFp8 ? 20 : 128;
     const uint32_t esz = t == kElemFp8 ? 2 : 3;
     const uint64_t n = (uint64_t)f.M * K;
-    const auto &T = fp8_tables();
 
     std::vector<std::array<uint64_t, 128>> part(host_threads() + 1);
     std::atomic<int> slot{0};
@@ -266,15 +278,8 @@ int64_t encode_fixed(const Splitter &S, const void *wv, const Shape &f, uint64_t
     });
     uint64_t hist[128] = {0};
     for (int s = 0; s < slot; s++) for (int k = 0; k < 128; k++) hist[k] += part[s][k];
-    int ord[128];
-    rank_symbols(hist, nsym, ord);
     uint8_t rank[128];
-    for (int r = 0; r < 128; r++) rank[ord[r]] = (uint8_t)std::min(r, 7);
-    for (uint32_t i = 0; i < kNpsym; i++) psym[i] = 0;
-    for (int r = 0; r < 7; r++) {
-        psym[r] = (uint16_t)(t == kElemFp8 ? T.hb2[ord[r]] : ord[r]);
-        psym[8 + r] = (uint16_t)(t == kElemFp8 ? T.lb2[ord[r]] : 0);
-    }
+    rank_and_psym(hist, t, 2, rank, psym);
 
     auto each_pos = [&](uint32_t b, uint32_t L, auto &&fn) {
         const uint32_t rb = b / f.CB, cb = b % f.CB;
@@ -411,6 +416,12 @@ extern "C" int64_t nwc_encode(const void *w, uint64_t n, uint32_t K, int elem, u
     Shape f((uint32_t)M, K, lay);
     if (lay == 2) return encode_fixed(S, w, f, K, t, psym, bases, hdr, data, data_cap, low);
     return encode_prefix(S, f, K, t, lay, psym, bases, hdr, data, data_cap, low);
+}
+
+extern "C" int nwc_encode_rank(const uint64_t *count, int elem, uint16_t *psym, uint8_t *rank) {
+    if (elem_type(elem) > 1 || elem_layout(elem) > 2) return -1;
+    rank_and_psym(count, elem_type(elem), elem_layout(elem), rank, psym);
+    return 0;
 }
 
 // 4096-entry decode table of layouts 0/1: for every 12-bit window the codes that are complete inside it (at most

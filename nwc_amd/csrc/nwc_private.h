@@ -18,6 +18,25 @@ int nwc_tokens(void *stream, const uint8_t *data, const uint32_t *bases, const u
                const uint16_t *bias, const float *scale, uint16_t *y, void *ws, uint64_t ws_bytes, uint64_t n, uint32_t K,
                int elem, uint32_t ntok);
 
+/* The encoder on the GPU (kern_encode.hip), in the order a caller runs them; w: the row-major source on the device.
+ * nwc_encode_supported: whether it takes the shape (else the host's nwc_encode).
+ * nwc_encode_hist adds the symbol counts of n weights to count[0..127] and, where fp8 input holds NaN, to count[128].
+ * nwc_encode_rank (host) turns the counts into psym[0..1023] (as nwc_encode) and rank[0..127].
+ * nwc_encode_sizes writes hdr[32 nb] and each block's bytes, and sets *over where a lane passes 255 words or exceptions.
+ * nwc_encode_write writes streams (block b at bases[b], a multiple of 8) and the raw plane; what it does not write of
+ * `data` and `low` (gaps, slack) the caller has zeroed.  0, -1, or a HIP error. */
+int nwc_encode_supported(uint64_t M, uint32_t K, int elem);
+int nwc_encode_hist(void *stream, const void *w, uint64_t n, int elem, uint64_t *count);
+int nwc_encode_rank(const uint64_t *count, int elem, uint16_t *psym, uint8_t *rank);
+int nwc_encode_sizes(void *stream, const void *w, uint64_t M, uint32_t K, int elem, const uint8_t *rank, uint8_t *hdr,
+                     uint32_t *size, uint32_t *over);
+int nwc_encode_write(void *stream, const void *w, uint64_t M, uint32_t K, int elem, const uint8_t *rank,
+                     const uint8_t *hdr, const uint32_t *bases, uint8_t *data, uint8_t *low);
+
+/* dst[to[b] + j] = src[from[b] + j] for every block b and j < size[b]; all multiples of 4. */
+int nwc_copy_spans(void *stream, const uint8_t *src, const int64_t *from, uint8_t *dst, const int64_t *to,
+                   const int64_t *size, uint32_t nb);
+
 #ifdef __cplusplus
 }
 #endif

@@ -237,18 +237,74 @@ def _encode(src, rows, cols, code):
                                 ptr(low))
         if length != -1:
             break
-    if length == -2:
-        raise ValueError("fp8 weights contain NaN")
-    if length == -3:
-        raise ValueError("layout 2 cannot code this matrix (a lane stream has more than 255 exceptions); "
-                         "use layout 0 or 1")
     if length < 0:
-        raise RuntimeError(f"nwc_encode failed ({length})")
+        raise _encode_error(length)
     lut = torch.empty(TAB_WORDS, dtype=torch.int32)
     lib.nwc_build_tab(ptr(freq), ptr(psym), code, ptr(lut))
     data = torch.zeros(length + DATA_SLACK, dtype=torch.uint8)
     data[:length] = buf[:length]
     return {"data": data, "bases": bases, "hdr": hdr, "lut": lut, "low": low}, length, geo
+
+
+def _encode_error(length):
+    """The exception of a nwc_encode failure code."""
+    if length == -2:
+        return ValueError("fp8 weights contain NaN")
+    if length == -3:
+        return ValueError("layout 2 cannot code this matrix (a lane stream has more than 255 exceptions); "
+                          "use layout 0 or 1")
+    return RuntimeError(f"nwc_encode failed ({length})")
+
+
+def _slot_stride(largest, blocks, layout, packed_len):
+    """The fixed-slot stride for blocks of at most `largest` stream bytes, or 0 to keep them packed: the slots would hold
+    more than SLOT_OVERHEAD times the bytes, or the stride passes the layout's SLOT_MAX."""
+    stride = -(-largest // 16) * 16
+    if not 0 < stride <= SLOT_MAX[layout] or blocks * stride > SLOT_OVERHEAD * packed_len \
+            or blocks * stride + SLOT_TAIL >= 1 << 31:
+        return 0
+    return stride
+
+
+def _encode_on_gpu(src, rows, cols, code):
+    """_encode on row-major source bits in GPU memory: the same bytes, made by the GPU (kern_encode.hip).  Returns the stored
+    tensors there, streams of layouts 0/1 already in fixed slots where _to_slots would move them, with their length,
+    geometry, packed bases and stride (None and 0: packed), and the host copy of the LUT."""
+    geo, dev, layout = _geometry(rows, cols, code), src.device, code >> 4
+    nb = geo.blocks
+    count = torch.zeros(129, dtype=torch.int64, device=dev)
+    call("nwc_encode_hist", stream(), ptr(src), rows * cols, code, ptr(count))
+    count = count.cpu()
+    if count[128]:
+        raise _encode_error(-2)
+    psym, rank = torch.empty(NPAIR, dtype=torch.int16), torch.empty(128, dtype=torch.uint8)
+    lib.nwc_encode_rank(ptr(count), code, ptr(psym), ptr(rank))
+    lut = torch.empty(TAB_WORDS, dtype=torch.int32)
+    lib.nwc_build_tab(None, ptr(psym), code, ptr(lut))
+    rank = rank.to(dev)
+    hdr = torch.empty(nb * HDR_BLOCK, dtype=torch.uint8, device=dev)
+    size = torch.zeros(nb + 1, dtype=torch.int32, device=dev)           # and the overflow flag
+    call("nwc_encode_sizes", stream(), ptr(src), rows, cols, code, ptr(rank), ptr(hdr), ptr(size), ptr(size) + 4 * nb)
+    size, over = size[:nb].long(), size[nb:].long()
+    held = (size + 7) // 8 * 8                                          # blocks begin at multiples of 8
+    ends = held.cumsum(0)
+    over, largest, total, last, last_held = torch.stack(
+        (over[0], size.max(), ends[-1], size[-1], held[-1])).tolist()
+    if over or total - last_held + last + 64 > _encoder_capacities(rows * cols, nb)[-1]:
+        raise _encode_error(-3 if over and layout == 2 else -1)
+    length = total + 64
+    packed = (ends - held).to(torch.int32)
+    stride = _slot_stride(largest, nb, layout, length + DATA_SLACK) if layout <= 1 and FIXED_SLOTS else 0
+    if stride:
+        data = torch.zeros(nb * stride + SLOT_TAIL, dtype=torch.uint8, device=dev)
+        bases = (torch.arange(nb, device=dev, dtype=torch.int64) * stride).to(torch.int32)
+    else:
+        data, bases = torch.zeros(length + DATA_SLACK, dtype=torch.uint8, device=dev), packed
+    low = torch.empty(geo.raw_bytes + RAW_SLACK, dtype=torch.uint8, device=dev)
+    low[geo.raw_bytes:].zero_()
+    call("nwc_encode_write", stream(), ptr(src), rows, cols, code, ptr(rank), ptr(hdr), ptr(bases), ptr(data), ptr(low))
+    stored = {"data": data, "bases": bases, "hdr": hdr, "lut": lut.to(dev), "low": low}
+    return stored, length, geo, packed if stride else None, stride, lut
 
 
 def _validate_streams(bases, hdr, data_len, layout, elem):
@@ -279,7 +335,13 @@ def _block_spans(bases, hdr):
 
 
 def _copy_spans(src, dst, src_start, dst_start, size, chunk=2048):
-    """dst[dst_start[b] + j] = src[src_start[b] + j] for every block b and j < size[b], a chunk of blocks at a time."""
+    """dst[dst_start[b] + j] = src[src_start[b] + j] for every block b and j < size[b] (all multiples of four): one kernel
+    on a GPU, a chunk of blocks at a time elsewhere."""
+    if src.is_cuda:
+        with torch.cuda.device(src.device):
+            call("nwc_copy_spans", stream(), ptr(src), ptr(src_start.contiguous()), ptr(dst), ptr(dst_start.contiguous()),
+                 ptr(size.contiguous()), size.numel())
+        return
     j = torch.arange(int(size.max()), device=src.device)
     for b0 in range(0, size.numel(), chunk):
         part = slice(b0, b0 + chunk)
@@ -303,26 +365,47 @@ class NWCWeight:
         kind = ELEMS[elem]
         layout = LAYOUT_DEFAULT[kind] if layout is None else int(layout)
         _check_layout(layout)
-        src, scale = self._source(w, kind, scale)
         self._shape(rows, cols, block, kind, layout)
-        stored, length, geo = _encode(src, rows, cols, self.code)
-        self._place(stored, scale, device, geo)
-        self.bytes = self._stored_bytes(length)
+        if not self._encode_there(w, scale, torch.device(device)):
+            src, scale = self._source(w, kind, scale)
+            stored, length, geo = _encode(src.cpu(), rows, cols, self.code)
+            self._place(stored, scale, device, geo)
+            self.bytes = self._stored_bytes(length)
         self._derive()
+
+    def _encode_there(self, w, scale, device):
+        """Encode on the GPU the matrix is placed on: w goes there once and the stored tensors never cross back.  False
+        where that does not serve: no GPU target, a shape the kernels do not take, graph capture (the sizes come back
+        to the host), or no room there for the uncompressed matrix next to the compressed one."""
+        if device.type != "cuda" or not lib.nwc_encode_supported(self.out_features, self.in_features, self.code) \
+                or torch.cuda.is_current_stream_capturing():
+            return False
+        try:
+            with torch.cuda.device(device):
+                src, scale = self._source(w.detach().to(device), self.elem, scale)
+                stored, length, geo, packed, stride, lut = _encode_on_gpu(src, self.out_features, self.in_features, self.code)
+                self._adopt(stored, scale, device, geo)
+                self._packed_len, self._packed, self._slot = length + DATA_SLACK, packed, stride
+                if self.layout <= 1 and SEQ_TABLE:
+                    self._seq_table = self._make_seq_table(lut)
+        except torch.OutOfMemoryError:
+            return False
+        self.bytes = self._stored_bytes(length)
+        return True
 
     @staticmethod
     def _source(w, kind, scale):
-        """Row-major source bits on the CPU and the fp32 row scale (fp8 only)."""
+        """Row-major source bits, where w is, and the fp32 row scale (fp8 only)."""
         if kind == ELEM_BF16:
             assert w.dtype == torch.bfloat16, "BF16 expected (elem='fp8' for fp8 weights)"
-            return w.detach().contiguous().cpu().view(torch.int16), None
+            return w.detach().contiguous().view(torch.int16), None
         if w.dtype == torch.float8_e4m3fn:
             if scale is None:
                 raise ValueError("fp8 weights need their per-row scale")
             codes = w
         else:
             codes, scale = quantize_fp8(w)
-        return codes.detach().contiguous().cpu().view(torch.uint8), scale.detach().float().contiguous()
+        return codes.detach().contiguous().view(torch.uint8), scale.detach().float().contiguous()
 
     def _shape(self, rows, cols, block, kind, layout):
         self.out_features, self.in_features = rows, cols
@@ -331,7 +414,7 @@ class NWCWeight:
         self.elem, self.layout = kind, layout
         self._slot, self._packed = 0, None
 
-    def _place(self, stored, scale, device, geo):
+    def _adopt(self, stored, scale, device, geo):
         for name in ("data", "bases", "hdr", "lut", "low"):
             setattr(self, name, stored[name].to(device))
         self.scale = None if scale is None else scale.float().to(device)
@@ -341,6 +424,9 @@ class NWCWeight:
         self.bytes_bf16 = 2 * self.n
         self.bytes_native = self.n + 4 * self.out_features if self.elem == ELEM_FP8 else 2 * self.n
         self._packed_len = self.data.numel()
+
+    def _place(self, stored, scale, device, geo):
+        self._adopt(stored, scale, device, geo)
         # (not inside HIP-graph capture: the move ends in a host read of two sums)
         if (self.layout <= 1 and FIXED_SLOTS and self.data.device.type == "cuda" and self.bases.numel()
                 and not torch.cuda.is_current_stream_capturing()):
@@ -354,9 +440,8 @@ class NWCWeight:
         it exactly)."""
         start, size = _block_spans(self.bases, self.hdr)
         nb = size.numel()
-        stride = -(-int(size.max()) // 16) * 16
-        if not 0 < stride <= SLOT_MAX[self.layout] or nb * stride > SLOT_OVERHEAD * self._packed_len \
-                or nb * stride + SLOT_TAIL >= 1 << 31:
+        stride = _slot_stride(int(size.max()), nb, self.layout, self._packed_len)
+        if not stride:
             return
         slots = torch.zeros(nb * stride + SLOT_TAIL, dtype=torch.uint8, device=self.data.device)
         first = torch.arange(nb, device=self.data.device, dtype=torch.int64) * stride
@@ -473,12 +558,14 @@ class NWCWeight:
             return None
         if self._seq_table is None:
             self._not_capturing("seq_table")
-            table = torch.empty(SEQ_TABLE_WORDS, dtype=torch.int32)
-            lut = self.lut.cpu().contiguous()
-            if lib.nwc_seq_table(ptr(lut), self.code, ptr(table)):
-                raise RuntimeError("nwc_seq_table failed")
-            self._seq_table = table.to(self.data.device)
+            self._seq_table = self._make_seq_table(self.lut.cpu().contiguous())
         return self._seq_table
+
+    def _make_seq_table(self, lut):
+        table = torch.empty(SEQ_TABLE_WORDS, dtype=torch.int32)
+        if lib.nwc_seq_table(ptr(lut), self.code, ptr(table)):
+            raise RuntimeError("nwc_seq_table failed")
+        return table.to(self.data.device)
 
     def token_bytes(self):
         """Bytes one token-path call reads: the compressed matrix, the row-index entries its plan uses (64 per block
