@@ -575,30 +575,58 @@ extern "C" int nwc_prefill_xbf16(void *stream, const uint8_t *data, const uint32
 
 namespace {
 
-// Small batches (kern_tokens.hip): `parts` workgroups per column block, one workgroup per CU in all (the decode table and
-// the activations are staged once a workgroup), with the waves that their LDS share and their rounds of row groups need;
-// the 13-bit table wherever it is given (the stored LUT's 16 KB less bought no wave that paid for its slow steps).
+// Small batches (kern_tokens.hip), one workgroup per CU (the decode table and the activations are staged once a workgroup)
+// with the waves that their LDS share and their rounds of tasks need; the 13-bit table wherever it is given (the stored
+// LUT's 16 KB less bought no wave that paid for its slow steps).  Where the activations of all column blocks and the
+// tasks' sums fit the LDS next to the waves, a workgroup may take whole rows and finish them (direct): no workspace and no
+// second kernel, 3.3 us.  The cheaper of the two by a model in sixteenths of 2.5 us: a round of tasks costs 16 for its
+// latency and one per task for the CU's throughput, each batch of activation loads after the first 4, the second kernel 21
+// (graph-timed, layout 0: 19456 x 2560 at 8 tokens
+// direct 24.9 us, split 27.2; 2560 x 4096 at 8 15.4 and 14.2, at 12, where the activations leave room for half the waves,
+// 22.6 and 14.4; 2560 x 9728 at 4 26.2 and 20.8; layout 2, 19456 x 2560 at 16 23.3 and 26.2).
 constexpr uint32_t kMaxTokens = 64;
 bool plan_tokens(const Shape &f, int elem, uint32_t T, int ncu, bool index, bool seq, TokensPlan &q, TokensArgs &p) {
     const int layout = elem_layout(elem);
-    const uint32_t units = f.groups(), nt = T <= 16u ? 1u : T <= 32u ? 2u : 4u, stride = elem_stride(elem);
-    if ((layout <= 1 && !index) || f.CB > (uint32_t)ncu) return false;
-    p.parts = std::min(units, (uint32_t)ncu / f.CB);
+    const uint32_t units = f.groups(), stride = elem_stride(elem), rows = layout ? 16u : 8u, n = (uint32_t)ncu;
+    if ((layout <= 1 && !index) || f.CB > n) return false;
     // a block's slot and the 16 bytes read past it, or the usual size of packed streams
     p.cap = layout == 2 ? 0u : stride ? stride / 4u + 4u : layout ? kSlotWords1s : kSlotWords2;
     p.Mu = f.Mp;
     q.seq13 = seq && layout <= 1;
     const uint32_t table = layout == 2 ? 0u : q.seq13 ? kSeqTableWords : kLutWords + 4u;
-    const uint32_t xs = nt * 16u * kTokensXRow * 4u, taken = xs + 4u * (table + kTokensOverrun) + 256u;
-    const uint32_t own = 4u * (layout == 0 ? kTokensTileWords + p.cap : layout == 1 ? p.cap : kTokensPatchWords);
-    if (taken + own > kLdsPerCu) return false;
-    const uint32_t fit = std::min(kTokensMaxWaves, (kLdsPerCu - taken) / own);
-    const uint32_t per = (units + p.parts - 1u) / p.parts, rounds = (per + fit - 1u) / fit;
-    const uint32_t W = (per + rounds - 1u) / rounds;
-    q.threads = 64u * W;
-    q.grid = p.parts * f.CB;
+    const uint32_t own = layout == 0 ? kTokensTileWords + p.cap : layout == 1 ? p.cap : kTokensPatchWords + kTokensExcWords;
     // layout 1: what a lane may read past the last wave's slot when its half's range ends before the other's
-    q.lds = xs + W * own + (layout == 1 ? kTokensOverrun * 4u : 0u);
+    const uint32_t extra = layout == 1 ? kTokensOverrun : 0u, lds = kLdsPerCu / 4u - 64u - table - extra;
+    struct Try {
+        uint32_t parts, xrow, xwords, sums, waves, rounds, cost;
+    };
+    auto attempt = [&](bool direct) {
+        Try t{};
+        t.parts = direct ? std::min(units, n) : std::min(units, n / f.CB);
+        const uint32_t most = (units + t.parts - 1u) / t.parts, tasks = most * (direct ? f.CB : 1u);
+        t.xrow = (direct ? f.CB : 1u) * (kCols / 2u) + 4u;
+        t.xwords = T * t.xrow;
+        t.sums = direct ? tasks * T * rows : 0u;
+        if ((uint64_t)T * t.xrow + (uint64_t)tasks * T * rows > lds && direct) return t;
+        const uint32_t left = lds - t.xwords - t.sums;
+        const uint32_t fit = t.xwords + t.sums + own > lds ? 0u : std::min(kTokensMaxWaves, left / own);
+        if (fit == 0) return t;
+        t.rounds = (tasks + fit - 1u) / fit;
+        t.waves = (tasks + t.rounds - 1u) / t.rounds;
+        const uint32_t batches = (T * (direct ? f.CB : 1u) + 4u * t.waves - 1u) / (4u * t.waves);   // of staging x
+        t.cost = 16u * t.rounds + tasks + 4u * (batches - 1u) + (direct ? 0u : 21u);
+        return t;
+    };
+    const Try d = attempt(true), s = attempt(false);
+    p.direct = d.rounds != 0 && (s.rounds == 0 || d.cost <= s.cost);
+    const Try &t = p.direct ? d : s;
+    if (t.rounds == 0) return false;
+    p.parts = t.parts;
+    p.xrow = t.xrow;
+    p.xwords = t.xwords;
+    q.threads = 64u * t.waves;
+    q.grid = t.parts * (p.direct ? 1u : f.CB);
+    q.lds = 4u * (t.xwords + t.waves * own + extra + t.sums);
     return true;
 }
 
@@ -608,7 +636,7 @@ extern "C" int nwc_tokens(void *stream, const uint8_t *data, const uint32_t *bas
                           const uint8_t *low, const uint16_t *row_index, const uint32_t *seq_table, const uint16_t *x,
                           uint32_t ldx, const uint16_t *bias, const float *scale, uint16_t *y, void *ws, uint64_t ws_bytes,
                           uint64_t n, uint32_t K, int elem, uint32_t ntok) {
-    if (!shape_ok(n, kBlock, K, elem) || ntok < 2 || ntok > kMaxTokens || ldx < K) return -1;
+    if (!shape_ok(n, kBlock, K, elem) || ntok < 2 || ntok > kMaxTokens || ldx < K || K < 8u) return -1;
     const int ncu = current_cus();
     if (ncu <= 0) return (int)hipErrorNoDevice;
     const int layout = elem_layout(elem);
@@ -616,14 +644,13 @@ extern "C" int nwc_tokens(void *stream, const uint8_t *data, const uint32_t *bas
     TokensPlan q;
     TokensArgs p{};
     if (!plan_tokens(f, elem, ntok, ncu, row_index != nullptr, seq_table != nullptr, q, p)) return -1;
-    if (4ull * f.CB * ntok * p.Mu > ws_bytes || ws == nullptr || ((uintptr_t)ws & 15u) != 0) return -1;
+    if (!p.direct && (4ull * f.CB * ntok * p.Mu > ws_bytes || ws == nullptr || ((uintptr_t)ws & 15u) != 0)) return -1;
     p.a = BlockArgs{data, bases, hdr, tab, low, nullptr, bias, scale, y, layout <= 1 ? row_index : nullptr, f.M, f.K, 1u,
                     0u, layout <= 1 ? seq_table : nullptr, elem_stride(elem)};
     p.x = x;
     p.part = (float *)ws;
     p.T = ntok;
     p.ldx = ldx;
-    p.vec = K % 8u == 0 && ldx % 8u == 0 && ((uintptr_t)x & 15u) == 0;
     return launch_tokens(layout, elem_type(elem), q, p, (hipStream_t)stream);
 }
 

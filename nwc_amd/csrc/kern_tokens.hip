@@ -2,23 +2,25 @@
 // without a BF16 copy of the matrix: y[t] = W x[t] (fp8: times the row scale) + bias, all layouts, fp32 accumulation,
 // one rounding to BF16.
 //
-// A workgroup keeps one 512-column block's activations (16, 32 or 64 tokens) and the decode table in LDS for its whole
-// life, and its waves work through row groups, one task (row group, column block) at a time: a wave decodes a block on
-// its two halves (layout 0: rows 0-3 and 4-7; layouts 1/2: super-chunks 0-7 and 8-15; from the row index) and multiplies
-// it by v_mfma_f32_16x16x32_bf16 (A: 16 rows x 32 columns, lane l row l & 15, columns 8 (l >> 4) .. + 7; B: the same
-// columns of 16 tokens).  Decoded weights reach the operand's lanes through LDS that belongs to the wave alone (layout 0:
-// the block's exponent bytes; layout 2: one super-chunk a half) or through lane permutes (layout 1); a wave requests its
-// next task's streams and raw bytes while it decodes, so after the first barrier no wave waits for another.
-// Each task's sums go to a workspace [column block][token][row]; k_tokens_finish adds the column blocks in order, so
-// equal inputs give equal bits.
+// A workgroup keeps the decode table and activations in LDS for its whole life, and its waves work through blocks, one
+// task (row group, column block) at a time: a wave decodes a block on its two halves (layout 0: rows 0-3 and 4-7; layouts
+// 1/2: super-chunks 0-7 and 8-15; from the row index) and multiplies it by v_mfma_f32_16x16x32_bf16 (A: 16 rows x 32
+// columns, lane l row l & 15, columns 8 (l >> 4) .. + 7; B: the same columns of 16 tokens).  Decoded weights reach the
+// operand's lanes through LDS that belongs to the wave alone (layout 0: the block's exponent bytes; layout 2: one
+// super-chunk a half) or through lane permutes (layout 1); a wave requests its next task's streams and raw bytes while it
+// decodes, so after the first barrier no wave waits for another.
+// Two ways of sharing the matrix out (abi.cpp plan_tokens): a workgroup has one column block of a run of row groups and
+// its sums go to a workspace [column block][token][row], which k_tokens_finish adds in order; or, where the activations
+// fit, all column blocks of its rows, whose sums it adds in LDS in order.  Either way equal inputs give equal bits.
 //
 // What bounds it: the LDS pipe (the decode's table reads, about 24k of 60k cycles a CU on 19456 x 2560) and the latency
 // of its chain, so the split aims at waves: a task of one block a wave keeps the LDS share of a wave at 6 KB (layout 0),
-// which lets 16 waves share a CU (8-9 with two row groups a wave: 19456 x 2560 at 16 tokens 34.6 us, now 28.7; two
-// interleaved cursors a lane instead 34.0; activations from L2 instead of LDS 38.4, at 64 tokens 82 instead of 42).
-// Against the temporary BF16 matrix and hipBLASLt, graph-timed with matrices out of the caches, layout 0, 32 tokens:
-// 6144 x 2560 18.3 against 34 us, 2560 x 4096 15.8 against 31, 19456 x 2560 31.0 against 87, 2560 x 9728 23.8 against
-// 43; layout 2 15.5 / 13.0 / 29.4 / 21.9 against 40 / 37 / 104 / 48.  The finish is 3.3 us of each.
+// which lets 16 waves share a CU (8-9 with two row groups a wave: 19456 x 2560 at 16 tokens 34.6 us, now 28.6; two
+// interleaved cursors a lane instead 34.0; activations from L2 instead of LDS 38.4, at 64 tokens 82 instead of 43).
+// Against the temporary BF16 matrix and hipBLASLt, graph-timed with matrices out of the caches, 32 tokens (4 tokens),
+// layout 0: 6144 x 2560 18.1 (14.2) against 34 us, 2560 x 4096 15.4 (13.6) against 31, 19456 x 2560 31.8 (24.6) against 87,
+// 2560 x 9728 23.0 (20.3) against 43; layout 1 17.9 / 18.2 / 31.6 / 23.7 against 36 / 32 / 100 / 48; layout 2 15.6 / 14.3 /
+// 29.3 / 21.6 against 40 / 37 / 104 / 48.  The second kernel is 3.3 us of a split product.
 #include "nwc_fixed.h"
 #include "nwc_launch.h"
 #include "nwc_prefix.h"
@@ -51,79 +53,90 @@ __device__ __forceinline__ void wave_lds_order() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// The column block's activations in LDS: token t's 512 columns from xs + t * kTokensXRow, zero past K and for tokens past
-// T.  Rows 4 banks apart, so that an operand read (16 tokens) meets no bank twice.  The first N chunks of 8 columns per
-// thread are requested early (issue); commit stores them and copies the rest.  Rows that are not made of whole aligned
-// chunks (p.vec false) are read value by value, which costs less than the two launches of a padded copy.
-template <int NT>
+// The activations in LDS: token t's columns (512 of one column block, or all of them) from xs + t * p.xrow, zero past K.
+// Rows 4 banks apart, so that an operand read (16 tokens) meets no bank twice.  The first N chunks of 8 columns per thread
+// are requested early (issue); commit stores them and copies the rest.  Rows that begin anywhere and end inside a chunk are
+// read as they are (x8_tail's way), which costs less than the two launches of a padded copy.
 struct StageX {
-    static constexpr uint32_t N = NT == 1 ? 4 : 8, TOTAL = NT * 16u * 64u;
+    static constexpr uint32_t N = 4;
     u32x4_t v[N];
-    __device__ __forceinline__ void load(const TokensArgs &p, uint32_t cb, uint32_t i0) {
+    uint32_t per, total, col0;                                   // chunks a row and in all, first column
+    __device__ __forceinline__ void load(const TokensArgs &p, uint32_t i0) {
         const uint32_t K = p.a.K;
-        if (p.vec) {
-#pragma unroll
-            for (uint32_t k = 0; k < N; k++) {
-                const uint32_t i = i0 + k * blockDim.x, t = i >> 6, col = cb * kCols + 8u * (i & 63u);
-                const bool in = t < p.T && col < K;
-                v[k] = *(const u32x4_t *)(p.x + (in ? (uint64_t)t * p.ldx + col : 0u));
-                if (!in) v[k] = u32x4_t{0u, 0u, 0u, 0u};
-            }
-            return;
-        }
 #pragma unroll
         for (uint32_t k = 0; k < N; k++) {
-            const uint32_t i = i0 + k * blockDim.x, t = i >> 6, col = cb * kCols + 8u * (i & 63u);
-            const uint16_t *row = p.x + (uint64_t)min(t, p.T - 1u) * p.ldx;
-#pragma unroll
-            for (uint32_t e = 0; e < 4; e++) {
-                const uint32_t c = col + 2u * e;
-                const uint32_t lo = row[min(c, K - 1u)], hi = row[min(c + 1u, K - 1u)];
-                v[k][e] = t < p.T ? (c < K ? lo : 0u) | (c + 1u < K ? hi << 16 : 0u) : 0u;
-            }
+            const uint32_t i = min(i0 + k * blockDim.x, total - 1u), t = i / per, col = col0 + 8u * (i - t * per);
+            v[k] = *(const u32x4_any *)(p.x + (uint64_t)t * p.ldx + min(col, K - 8u));
         }
     }
-    __device__ __forceinline__ void store(uint32_t *xs, uint32_t i0) const {
+    __device__ __forceinline__ void store(uint32_t *xs, const TokensArgs &p, uint32_t i0) const {
 #pragma unroll
         for (uint32_t k = 0; k < N; k++) {
-            const uint32_t i = i0 + k * blockDim.x;
-            if (i < TOTAL) *(u32x4_t *)(xs + (i >> 6) * kTokensXRow + 4u * (i & 63u)) = v[k];
+            const uint32_t i = i0 + k * blockDim.x, t = i / per, K = p.a.K, col = col0 + 8u * (i - t * per);
+            if (i >= total) continue;
+            uint32_t w[4] = {v[k].x, v[k].y, v[k].z, v[k].w};
+            if (K & 7u) shift_down<4>(w, col - min(col, K - 8u));
+            const uint32_t keep = col < K ? ~0u : 0u;
+            *(uint4 *)(xs + t * p.xrow + 4u * (i - t * per)) = make_uint4(w[0] & keep, w[1] & keep, w[2] & keep, w[3] & keep);
         }
     }
-    __device__ __forceinline__ void issue(const TokensArgs &p, uint32_t cb) { load(p, cb, threadIdx.x); }
-    __device__ __forceinline__ void commit(uint32_t *xs, const TokensArgs &p, uint32_t cb) {
-        store(xs, threadIdx.x);
-        for (uint32_t i0 = threadIdx.x + N * blockDim.x; i0 < TOTAL; i0 += N * blockDim.x) {
-            load(p, cb, i0);
-            store(xs, i0);
+    __device__ __forceinline__ void issue(const TokensArgs &p, uint32_t cb, uint32_t blocks) {
+        per = 64u * blocks;
+        total = p.T * per;
+        col0 = cb * kCols;
+        load(p, threadIdx.x);
+    }
+    __device__ __forceinline__ void commit(uint32_t *xs, const TokensArgs &p) {
+        store(xs, p, threadIdx.x);
+        for (uint32_t i0 = threadIdx.x + N * blockDim.x; i0 < total; i0 += N * blockDim.x) {
+            load(p, i0);
+            store(xs, p, i0);
         }
     }
 };
 
-// A task's sums: lane l holds rows row0 + 4 (l >> 4) .. + 3 for tokens 16 j + (l & 15).
-template <int NT>
-__device__ __forceinline__ void store_part(const TokensArgs &p, uint32_t cb, uint32_t row0, const f32x4_t (&acc)[NT]) {
-    const uint32_t lane = threadIdx.x & 63u;
-    float *o = p.part + (uint64_t)cb * p.T * p.Mu + row0 + 4u * (lane >> 4);
+// A wave's tasks: t = wave, wave + waves, ... < n of its workgroup's.  A workgroup has a run of row groups ("units"), and
+// either one column block of them (blockIdx = part * CB + cb), its sums going to the workspace, or, `direct`, all of their
+// column blocks, whose sums it adds in LDS and finishes itself.
+struct TokensTasks {
+    uint32_t CB, u0, cb0, n, step, t;
+    bool direct;
+    __device__ __forceinline__ void init(const TokensArgs &p, const Shape &f) {
+        CB = f.CB;
+        direct = p.direct;
+        const uint32_t part = direct ? blockIdx.x : blockIdx.x / CB, units = f.groups();
+        cb0 = direct ? 0u : blockIdx.x - part * CB;
+        u0 = (uint32_t)((uint64_t)part * units / p.parts);
+        n = ((uint32_t)((uint64_t)(part + 1u) * units / p.parts) - u0) * (direct ? CB : 1u);
+        step = blockDim.x >> 6;
+        t = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    }
+    // task i's unit and column block (past the last: the last again)
+    __device__ __forceinline__ void at(uint32_t i, uint32_t &unit, uint32_t &cb) const {
+        i = min(i, n - 1u);
+        const uint32_t q = direct ? i / CB : i;
+        unit = u0 + q;
+        cb = direct ? i - q * CB : cb0;
+    }
+};
+
+// A task's sums: lane l holds rows 4 (l >> 4) .. + 3 of the R rows of its unit for tokens 16 j + (l & 15).
+template <int NT, int R>
+__device__ __forceinline__ void store_part(const TokensArgs &p, const TokensTasks &w, uint32_t unit, float *sums,
+                                           const f32x4_t (&acc)[NT]) {
+    const uint32_t lane = threadIdx.x & 63u, m = 4u * (lane >> 4);
+    if (m >= (uint32_t)R) return;
 #pragma unroll
     for (int j = 0; j < NT; j++) {
         const uint32_t t = 16u * j + (lane & 15u);
-        if (t < p.T) *(f32x4_t *)(o + (uint64_t)t * p.Mu) = acc[j];
+        if (t >= p.T) break;
+        if (w.direct) *(f32x4_t *)(sums + (w.t * p.T + t) * R + m) = acc[j];
+        else *(f32x4_t *)(p.part + ((uint64_t)w.cb0 * p.T + t) * p.Mu + unit * R + m) = acc[j];
     }
 }
 
-// y from the column blocks' sums, in order.
-__global__ void __launch_bounds__(256) k_tokens_finish(TokensArgs p, uint32_t CB) {
-    const BlockArgs &a = p.a;
-    const uint32_t q = p.Mu / 4u, i = blockIdx.x * 256u + threadIdx.x;
-    if (i >= p.T * q) return;
-    const uint32_t t = i / q, m = 4u * (i - t * q);
-    if (m >= a.M) return;
-    const float *src = p.part + (uint64_t)t * p.Mu + m;
-    const uint64_t step = (uint64_t)p.T * p.Mu;
-    f32x4_t v = *(const f32x4_t *)src;
-#pragma unroll 4
-    for (uint32_t s = 1; s < CB; s++) v += *(const f32x4_t *)(src + s * step);
+// Rows m .. m + 3 of token t: scale, bias, one rounding.
+__device__ __forceinline__ void finish4(const BlockArgs &a, uint32_t t, uint32_t m, const f32x4_t &v) {
     uint32_t h[4];
 #pragma unroll
     for (uint32_t e = 0; e < 4; e++) {
@@ -143,19 +156,33 @@ __global__ void __launch_bounds__(256) k_tokens_finish(TokensArgs p, uint32_t CB
     }
 }
 
-// A wave's place in the grid: workgroup blockIdx = part * CB + cb holds column block cb, and its wave w takes row groups
-// ("units") part * W + w, + parts * W, ...
-struct TokensWave {
-    uint32_t cb, unit, step, units;
-};
-__device__ __forceinline__ TokensWave tokens_wave(const TokensArgs &p, const Shape &f) {
-    TokensWave w;
-    const uint32_t part = blockIdx.x / f.CB, W = blockDim.x >> 6;
-    w.cb = blockIdx.x - part * f.CB;
-    w.unit = part * W + (threadIdx.x >> 6);
-    w.step = p.parts * W;
-    w.units = f.groups();
-    return w;
+// The direct workgroup's rows from its tasks' sums in LDS, column blocks in order.
+template <int R>
+__device__ __forceinline__ void finish_direct(const TokensArgs &p, const TokensTasks &w, const float *sums) {
+    __syncthreads();
+    const uint32_t units = w.n / w.CB, q = R / 4u;
+    for (uint32_t i = threadIdx.x; i < units * p.T * q; i += blockDim.x) {
+        const uint32_t ut = i / q, u = ut / p.T, t = ut - u * p.T, m = 4u * (i - ut * q);
+        if ((w.u0 + u) * R + m >= p.a.M) continue;
+        const float *src = sums + (u * w.CB * p.T + t) * R + m;
+        f32x4_t v = *(const f32x4_t *)src;
+        for (uint32_t c = 1; c < w.CB; c++) v += *(const f32x4_t *)(src + c * p.T * R);
+        finish4(p.a, t, (w.u0 + u) * R + m, v);
+    }
+}
+
+// y from the column blocks' sums, in order.
+__global__ void __launch_bounds__(256) k_tokens_finish(TokensArgs p, uint32_t CB) {
+    const uint32_t q = p.Mu / 4u, i = blockIdx.x * 256u + threadIdx.x;
+    if (i >= p.T * q) return;
+    const uint32_t t = i / q, m = 4u * (i - t * q);
+    if (m >= p.a.M) return;
+    const float *src = p.part + (uint64_t)t * p.Mu + m;
+    const uint64_t step = (uint64_t)p.T * p.Mu;
+    f32x4_t v = *(const f32x4_t *)src;
+#pragma unroll 4
+    for (uint32_t s = 1; s < CB; s++) v += *(const f32x4_t *)(src + s * step);
+    finish4(p.a, t, m, v);
 }
 
 // ---------------------------------------------------------------------------------------------------------------
@@ -215,24 +242,21 @@ __global__ void __launch_bounds__(kTokensMaxWaves * 64) k_tokens0(TokensArgs p) 
     const BlockArgs &a = p.a;
     __shared__ LutT<PEEK> s;
     extern __shared__ __attribute__((aligned(16))) uint32_t dyn[];
-    const uint32_t tid = threadIdx.x, lane = tid & 63u, wv = tid >> 6, L = tid & 31u, h = lane >> 5;
-    const uint32_t r8 = lane & 7u, far = (lane >> 3) & 1u, c4 = lane >> 4;
+    const uint32_t lane = threadIdx.x & 63u, L = threadIdx.x & 31u, h = lane >> 5;
+    const uint32_t r8 = lane & 7u, far = (lane >> 3) & 1u, i16 = lane & 15u, c4 = lane >> 4;
     const Shape f(a.M, a.K, 0);
-    TokensWave w = tokens_wave(p, f);
-    const uint32_t cols = min(kCols, f.K16 - w.cb * kCols);      // coded columns of the block
-    const bool col_ok = 16u * L < cols;
+    TokensTasks w;
+    w.init(p, f);
     const uint32_t tcol = 128u * far + 16u * c4;                  // operand columns of step j: + 64 (j & 1) + 256 (j >> 1)
     auto step_col = [](uint32_t j) { return 64u * (j & 1u) + 256u * (j >> 1); };
-    auto block_of = [&](uint32_t unit) { return min(unit, w.units - 1u) * f.CB + w.cb; };
-    auto header = [&](uint32_t unit) { return (uint32_t)a.hdr[(uint64_t)block_of(unit) * kHdrBytes + L]; };
+    auto cols_of = [&](uint32_t cb) { return min(kCols, f.K16 - cb * kCols); };      // coded columns of a block
     // lanes past the coded columns have no stream: they decode the block's first lane's rows, for nothing
-    auto part_at = [&](uint32_t unit) {
-        const uint32_t P = part_start(a, block_of(unit), 2u * h, L);
-        return col_ok ? P : 0u;
+    auto part_at = [&](uint32_t unit, uint32_t cb) {
+        const uint32_t P = part_start(a, unit * f.CB + cb, 2u * h, L);
+        return 16u * L < cols_of(cb) ? P : 0u;
     };
-    auto raw_at = [&](uint32_t unit, uint32_t j) {
-        const uint32_t row = min(min(unit, w.units - 1u) * 8u + r8, a.M - 1u);
-        const uint32_t col = min(w.cb * kCols + tcol + step_col(j), f.K16 - 16u);
+    auto raw_at = [&](uint32_t unit, uint32_t cb, uint32_t j) {
+        const uint32_t row = min(unit * 8u + r8, a.M - 1u), col = min(cb * kCols + tcol + step_col(j), f.K16 - 16u);
         if constexpr (ELEM == kElemFp8) {
             const uint2 v = ldnt2(a.low + (row * (f.K16 / 2u) + col / 2u));
             return make_uint4(v.x, v.y, 0u, 0u);
@@ -240,34 +264,42 @@ __global__ void __launch_bounds__(kTokensMaxWaves * 64) k_tokens0(TokensArgs p) 
             return ldnt4(a.low + (row * f.K16 + col));
         }
     };
-    uint32_t *xs = dyn, *tile = dyn + NT * 16u * kTokensXRow + wv * (kTokensTileWords + p.cap), *slot = tile + kTokensTileWords;
+    uint32_t *xs = dyn, *tile = dyn + p.xwords + w.t * (kTokensTileWords + p.cap), *slot = tile + kTokensTileWords;
+    float *sums = (float *)(dyn + p.xwords + w.step * (kTokensTileWords + p.cap));
     TabStage<PEEK> Q;
     Q.issue(a);
-    const uint32_t n = header(w.unit);
-    StageX<NT> X;
-    X.issue(p, w.cb);
+    uint32_t unit, cb, un, cn;
+    w.at(w.t, unit, cb);
+    w.at(w.t + w.step, un, cn);
+    const uint32_t n = a.hdr[(uint64_t)(unit * f.CB + cb) * kHdrBytes + L];
+    StageX X;
+    X.issue(p, w.cb0, w.direct ? f.CB : 1u);
     BlockStream<2> B;
-    B.request(a, block_of(w.unit), n, p.cap);
-    uint32_t nn = header(w.unit + w.step), P = part_at(w.unit);
+    B.request(a, unit * f.CB + cb, n, p.cap);
+    uint32_t nn = a.hdr[(uint64_t)(un * f.CB + cn) * kHdrBytes + L], P = part_at(unit, cb);
     Q.commit(s);
-    X.commit(xs, p, w.cb);
+    X.commit(xs, p);
     Q.finish(s, a);
     B.store(slot);
     __syncthreads();
     // the first task's raw bytes only now: nothing needs them before its decode is done
     uint4 raw[4];
 #pragma unroll
-    for (uint32_t j = 0; j < 4; j++) raw[j] = raw_at(w.unit, j);
-    const uint32_t keep = col_ok ? ~0u : 0u;
+    for (uint32_t j = 0; j < 4; j++) raw[j] = raw_at(unit, cb, j);
     uint32_t *mine = tile + 4u * h * kTokensTileRow + 4u * L;
     const uint32_t *er = tile + r8 * kTokensTileRow + tcol / 4u;
-    const uint32_t *xr = xs + (lane & 15u) * kTokensXRow + 8u * c4;
-    for (; w.unit < w.units; w.unit += w.step) {
-        const uint32_t start = col_ok ? B.start : (B.base & 15u) >> 2, base = B.base, from = P;
-        const bool fits = B.fits;
-        B.request(a, block_of(w.unit + w.step), nn, p.cap);
-        P = part_at(w.unit + w.step);
-        nn = header(w.unit + 2u * w.step);
+    uint32_t xr[NT];
+#pragma unroll
+    for (int t = 0; t < NT; t++) xr[t] = min(16u * t + i16, p.T - 1u) * p.xrow + 8u * c4;
+    for (; w.t < w.n; w.t += w.step) {
+        const uint32_t cols = cols_of(cb), base = B.base, from = P;
+        const bool fits = B.fits, col_ok = 16u * L < cols;
+        const uint32_t start = col_ok ? B.start : (B.base & 15u) >> 2, keep = col_ok ? ~0u : 0u;
+        uint32_t u2, c2;
+        w.at(w.t + 2u * w.step, u2, c2);
+        B.request(a, un * f.CB + cn, nn, p.cap);
+        P = part_at(un, cn);
+        nn = a.hdr[(uint64_t)(u2 * f.CB + c2) * kHdrBytes + L];
         if (fits) tokens_decode0<ELEM>(s, slot + start, from, keep, mine);
         else tokens_decode0<ELEM>(s, (const uint32_t *)(a.data + (base & ~15u)) + start, from, keep, mine);
         wave_lds_order();
@@ -275,6 +307,7 @@ __global__ void __launch_bounds__(kTokensMaxWaves * 64) k_tokens0(TokensArgs p) 
         f32x4_t acc[NT], acc_far[NT];
 #pragma unroll
         for (int t = 0; t < NT; t++) acc[t] = acc_far[t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+        const uint32_t *xc = xs + (w.direct ? cb * (kCols / 2u) : 0u);
         // all steps, also where the block has fewer columns: x is zero there and the weights are masked to +0
 #pragma unroll
         for (uint32_t j = 0; j < 4; j++) {
@@ -285,10 +318,10 @@ __global__ void __launch_bounds__(kTokensMaxWaves * 64) k_tokens0(TokensArgs p) 
                                         perm(e.y, rw.y, 0x05010400u) & in, perm(e.y, rw.y, 0x07030602u) & in);
             const bf16x8_t w1 = operand(perm(e.z, rw.z, 0x05010400u) & in, perm(e.z, rw.z, 0x07030602u) & in,
                                         perm(e.w, rw.w, 0x05010400u) & in, perm(e.w, rw.w, 0x07030602u) & in);
-            raw[j] = raw_at(w.unit + w.step, j);
+            raw[j] = raw_at(un, cn, j);
 #pragma unroll
             for (int t = 0; t < NT; t++) {
-                const uint32_t *x = xr + t * 16u * kTokensXRow + step_col(j) / 2u;
+                const uint32_t *x = xc + xr[t] + step_col(j) / 2u;
                 acc[t] = mfma(w0, operand(*(const uint4 *)x), acc[t]);
                 acc_far[t] = mfma(w0, operand(*(const uint4 *)(x + 64)), acc_far[t]);
                 acc[t] = mfma(w1, operand(*(const uint4 *)(x + 4)), acc[t]);
@@ -305,8 +338,13 @@ __global__ void __launch_bounds__(kTokensMaxWaves * 64) k_tokens0(TokensArgs p) 
                 swap32(u, v);                                    // v, lanes 0-31: acc_far's lanes 32-63
                 acc[t][e] += __uint_as_float(v);
             }
-        if (h == 0u) store_part<NT>(p, w.cb, w.unit * 8u, acc);
+        store_part<NT, 8>(p, w, unit, sums, acc);
+        unit = un;
+        cb = cn;
+        un = u2;
+        cn = c2;
     }
+    if (w.direct) finish_direct<8>(p, w, sums);
 }
 
 // ---------------------------------------------------------------------------------------------------------------
@@ -316,17 +354,16 @@ __global__ void __launch_bounds__(kTokensMaxWaves * 64) k_tokens0(TokensArgs p) 
 __device__ __forceinline__ uint32_t from_lane(uint32_t idx4, uint32_t v) {
     return (uint32_t)__builtin_amdgcn_ds_bpermute((int)idx4, (int)v);
 }
-// products of one super-chunk pair (half 0's chunk i, half 1's chunk 8 + i of the column block)
+// products of one super-chunk pair (half 0's chunk i, half 1's chunk 8 + i of the column block); xr: the lane's place in
+// each 16 tokens' rows
 template <int NT>
-__device__ __forceinline__ void chunk_products(bf16x8_t w0, bf16x8_t w1, bool two, const uint32_t *xr, uint32_t i,
-                                               f32x4_t (&acc)[NT]) {
+__device__ __forceinline__ void chunk_products(bf16x8_t w0, bf16x8_t w1, bool two, const uint32_t *xc, const uint32_t (&xr)[NT],
+                                               uint32_t i, f32x4_t (&acc)[NT]) {
 #pragma unroll
-    for (int j = 0; j < NT; j++)
-        acc[j] = mfma(w0, operand(*(const uint4 *)(xr + j * 16u * kTokensXRow + 16u * i)), acc[j]);
+    for (int j = 0; j < NT; j++) acc[j] = mfma(w0, operand(*(const uint4 *)(xc + xr[j] + 16u * i)), acc[j]);
     if (two) {
 #pragma unroll
-        for (int j = 0; j < NT; j++)
-            acc[j] = mfma(w1, operand(*(const uint4 *)(xr + j * 16u * kTokensXRow + 16u * (i + 8u))), acc[j]);
+        for (int j = 0; j < NT; j++) acc[j] = mfma(w1, operand(*(const uint4 *)(xc + xr[j] + 16u * (i + 8u))), acc[j]);
     }
 }
 
@@ -353,7 +390,7 @@ __device__ __forceinline__ void chunk_operands(const uint32_t (&e1)[4], const ui
 template <int ELEM, int NT, bool FULL, bool GLOBAL, class Tab>
 __device__ __forceinline__ void tokens_chunks1(const Tab &s, const uint32_t *lane_words, uint32_t P0, const uint8_t *low,
                                                uint32_t nsc, const Coord1 &c, const Coord1 &cn, uint32_t sc0, uint4 (&ring)[4],
-                                               const uint32_t *xr, f32x4_t (&acc)[NT]) {
+                                               const uint32_t *xc, const uint32_t (&xr)[NT], f32x4_t (&acc)[NT]) {
     const uint32_t lane = threadIdx.x & 63u, from = 4u * (4u * (lane & 15u) + (lane >> 4));
     Seq<ELEM> S;
     S.init_at(lane_words, P0);
@@ -364,7 +401,7 @@ __device__ __forceinline__ void tokens_chunks1(const Tab &s, const uint32_t *lan
             bf16x8_t w0, w1;
             if (!GLOBAL || sc0 + i < nsc) row_codes(S, s, e1, e2);
             chunk_operands(e1, e2, ring[i & 3u], from, w0, w1);
-            chunk_products<NT>(w0, w1, FULL || i + 8u < nsc, xr, i, acc);
+            chunk_products<NT>(w0, w1, FULL || i + 8u < nsc, xc, xr, i, acc);
         }
         ring[i & 3u] = i < 4u ? raw1<ELEM>(low, c, sc0 + i + 4u) : raw1<ELEM>(low, cn, sc0 + i - 4u);
     }
@@ -375,78 +412,125 @@ __global__ void __launch_bounds__(kTokensMaxWaves * 64) k_tokens1(TokensArgs p) 
     const BlockArgs &a = p.a;
     __shared__ LutT<PEEK> s;
     extern __shared__ __attribute__((aligned(16))) uint32_t dyn[];
-    const uint32_t tid = threadIdx.x, lane = tid & 63u, wv = tid >> 6, L = tid & 31u, h = lane >> 5;
+    const uint32_t lane = threadIdx.x & 63u, L = threadIdx.x & 31u, h = lane >> 5;
     const Shape f(a.M, a.K, 1);
-    TokensWave w = tokens_wave(p, f);
-    auto coord = [&](uint32_t unit) { return coord1<ELEM>(min(unit, w.units - 1u) * f.CB + w.cb, 0u, f, L); };
-    auto header = [&](uint32_t unit) {
-        return (uint32_t)a.hdr[(uint64_t)(min(unit, w.units - 1u) * f.CB + w.cb) * kHdrBytes + L];
-    };
-    uint32_t *xs = dyn, *slot = dyn + NT * 16u * kTokensXRow + wv * p.cap;
+    TokensTasks w;
+    w.init(p, f);
+    auto coord = [&](uint32_t unit, uint32_t cb) { return coord1<ELEM>(unit * f.CB + cb, 0u, f, L); };
+    auto nsc_of = [&](uint32_t cb) { return cb == f.CB - 1u ? f.nsl : 16u; };
+    // a half without super-chunks of its own decodes the block's first ones again, for nothing
+    auto part_at = [&](uint32_t b, uint32_t cb) { return part_start(a, b, 8u * h < nsc_of(cb) ? 2u * h : 0u, L); };
+    uint32_t *xs = dyn, *slot = dyn + p.xwords + w.t * p.cap;
+    float *sums = (float *)(dyn + p.xwords + w.step * p.cap + kTokensOverrun);
     TabStage<PEEK> Q;
     Q.issue(a);
-    Coord1 c = coord(w.unit);
-    const uint32_t n = header(w.unit);
-    StageX<NT> X;
-    X.issue(p, w.cb);
+    uint32_t unit, cb, un, nb;
+    w.at(w.t, unit, cb);
+    w.at(w.t + w.step, un, nb);
+    Coord1 c = coord(unit, cb);
+    const uint32_t n = a.hdr[(uint64_t)c.b * kHdrBytes + L];
+    StageX X;
+    X.issue(p, w.cb0, w.direct ? f.CB : 1u);
     BlockStream<4> B;
     B.request(a, c.b, n, p.cap);
-    // a half without super-chunks of its own decodes the block's first ones again, for nothing
-    const uint32_t nsc = w.cb == f.CB - 1u ? f.nsl : 16u, part = 8u * h < nsc ? 2u * h : 0u;
-    uint32_t P0 = part_start(a, c.b, part, L), nn = header(w.unit + w.step);
+    uint32_t P0 = part_at(c.b, cb), nn = a.hdr[(uint64_t)(un * f.CB + nb) * kHdrBytes + L];
     Q.commit(s);
-    X.commit(xs, p, w.cb);
+    X.commit(xs, p);
     Q.finish(s, a);
     B.store(slot);
     uint4 ring[4];
 #pragma unroll
     for (uint32_t i = 0; i < 4; i++) ring[i] = raw1<ELEM>(a.low, c, 8u * h + i);
     __syncthreads();
-    const uint32_t *xr = xs + (lane & 15u) * kTokensXRow + 4u * (lane >> 4);
-    for (; w.unit < w.units; w.unit += w.step) {
-        const uint32_t start = B.start, base = B.base, P = P0;
+    uint32_t xr[NT];
+#pragma unroll
+    for (int j = 0; j < NT; j++) xr[j] = min(16u * j + (lane & 15u), p.T - 1u) * p.xrow + 4u * (lane >> 4);
+    for (; w.t < w.n; w.t += w.step) {
+        const uint32_t start = B.start, base = B.base, P = P0, nsc = nsc_of(cb);
         const bool fits = B.fits;
-        const Coord1 cn = coord(w.unit + w.step);
+        const Coord1 cn = coord(un, nb);
+        uint32_t u2, b2;
+        w.at(w.t + 2u * w.step, u2, b2);
         B.request(a, cn.b, nn, p.cap);
-        P0 = part_start(a, cn.b, part, L);
-        nn = header(w.unit + 2u * w.step);
+        P0 = part_at(cn.b, nb);
+        nn = a.hdr[(uint64_t)(u2 * f.CB + b2) * kHdrBytes + L];
         f32x4_t acc[NT];
 #pragma unroll
         for (int j = 0; j < NT; j++) acc[j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+        const uint32_t *xc = xs + (w.direct ? cb * (kCols / 2u) : 0u);
         if (fits && nsc == 16u)
-            tokens_chunks1<ELEM, NT, true, false>(s, slot + start, P, a.low, nsc, c, cn, 8u * h, ring, xr, acc);
+            tokens_chunks1<ELEM, NT, true, false>(s, slot + start, P, a.low, nsc, c, cn, 8u * h, ring, xc, xr, acc);
         else if (fits)
-            tokens_chunks1<ELEM, NT, false, false>(s, slot + start, P, a.low, nsc, c, cn, 8u * h, ring, xr, acc);
+            tokens_chunks1<ELEM, NT, false, false>(s, slot + start, P, a.low, nsc, c, cn, 8u * h, ring, xc, xr, acc);
         else
             tokens_chunks1<ELEM, NT, false, true>(s, (const uint32_t *)(a.data + (base & ~15u)) + start, P, a.low, nsc, c, cn,
-                                                  8u * h, ring, xr, acc);
+                                                  8u * h, ring, xc, xr, acc);
         wave_lds_order();
         B.store(slot);
         wave_lds_order();
-        store_part<NT>(p, w.cb, w.unit * 16u, acc);
+        store_part<NT, 16>(p, w, unit, sums, acc);
         c = cn;
+        unit = un;
+        cb = nb;
+        un = u2;
+        nb = b2;
     }
+    if (w.direct) finish_direct<16>(p, w, sums);
 }
 
 // ---------------------------------------------------------------------------------------------------------------
 // Layout 2: the same fragment order without streams.  A super-chunk pair's 2 x 16 rows x 32 columns go through the
 // wave's LDS patch (row r's 16-byte piece q at place q ^ (r >> 2), so that neither the writes by lane nor the reads by
 // row meet in a bank), where the lanes' exceptions replace the planes' zeros before the operands are read.
+// A block's exception entries on their way into the wave's LDS, a task ahead; `fits`: else they are read from memory.
 template <int ELEM>
-struct ExcCursor {                                               // a lane's next exception: position (0..255) and BF16 bits
-    const uint8_t *ep;
-    uint32_t left, pos, bits;
-    __device__ __forceinline__ void load() {
-        pos = 0xFFFFu;
-        bits = 0u;
-        if (left) {
-            pos = ep[0];
-            if constexpr (ELEM == kElemFp8) bits = __float_as_uint(e4m3_to_f32(ep[1])) >> 16;     // exact
-            else bits = (uint32_t)ep[1] | (uint32_t)ep[2] << 8;
+struct ExcStream {
+    static constexpr uint32_t N = kTokensExcWords / 64u, SIZE = ELEM == kElemFp8 ? 2 : 3;
+    typedef __attribute__((aligned(1))) uint32_t any32;
+    uint32_t v[N], n, first, bytes, base;                        // of the lane: entries, the first one's byte
+    bool fits;
+    __device__ __forceinline__ void request(const BlockArgs &a, uint32_t b, uint32_t cnt) {
+        const uint32_t lane = threadIdx.x & 63u, incl = half_scan_incl(cnt, lane & 31u);
+        n = cnt;
+        first = (incl - cnt) * SIZE;
+        bytes = __builtin_amdgcn_readlane(incl, 31) * SIZE;
+        base = a.bases[b];
+        fits = bytes <= kTokensExcWords * 4u && bytes >= 4u;
+        // a word that would pass the last entry is read up to three bytes early and moved down: nothing past it is read
+        if (fits) {
+#pragma unroll
+            for (uint32_t k = 0; k < N; k++)
+                if (256u * k < bytes) v[k] = *(const any32 *)(a.data + base + min(4u * (lane + 64u * k), bytes - 4u));
         }
     }
+    __device__ __forceinline__ void store(uint32_t *slot) const {
+        if (!fits) return;
+        const uint32_t lane = threadIdx.x & 63u;
+#pragma unroll
+        for (uint32_t k = 0; k < N; k++) {
+            const uint32_t at = 4u * (lane + 64u * k);
+            if (at < bytes) slot[at / 4u] = v[k] >> (8u * (at - min(at, bytes - 4u)));
+        }
+    }
+};
+// A lane's next exception: position (0..255; 0xFFFF: none) and BF16 bits, from LDS or, `mem` set, from memory.
+template <int ELEM>
+struct ExcCursor {
+    const uint8_t *lds, *mem;
+    uint32_t at, left, pos, bits;
+    __device__ __forceinline__ void load() {
+        constexpr uint32_t SIZE = ExcStream<ELEM>::SIZE;
+        pos = 0xFFFFu;
+        if (left == 0u) return;
+        uint32_t e[3];
+#pragma unroll
+        for (uint32_t i = 0; i < SIZE; i++) e[i] = mem ? mem[at + i] : lds[at + i];
+        pos = e[0];
+        if constexpr (ELEM == kElemFp8) bits = __float_as_uint(e4m3_to_f32(e[1])) >> 16;     // exact
+        else bits = e[1] | e[2] << 8;
+    }
     __device__ __forceinline__ void next() {
-        ep += ELEM == kElemFp8 ? 2 : 3;
+        at += ExcStream<ELEM>::SIZE;
         left--;
         load();
     }
@@ -456,45 +540,62 @@ template <int ELEM, int NT>
 __global__ void __launch_bounds__(kTokensMaxWaves * 64) k_tokens2(TokensArgs p) {
     const BlockArgs &a = p.a;
     extern __shared__ __attribute__((aligned(16))) uint32_t dyn[];
-    const uint32_t tid = threadIdx.x, lane = tid & 63u, wv = tid >> 6, L = tid & 31u, h = lane >> 5;
+    const uint32_t lane = threadIdx.x & 63u, L = threadIdx.x & 31u, h = lane >> 5;
     const uint32_t i16 = lane & 15u, c4 = lane >> 4;
     const Shape f(a.M, a.K, 2);
-    TokensWave w = tokens_wave(p, f);
+    TokensTasks w;
+    w.init(p, f);
     const RankTab tab{a.lut[0], a.lut[1], a.lut[2], a.lut[3]};
     const uint8_t *rplane = a.low + f.nib2_bytes();
-    const uint32_t nsc = w.cb == f.CB - 1u ? f.nsl : 16u;
+    auto nsc_of = [&](uint32_t cb) { return cb == f.CB - 1u ? f.nsl : 16u; };
     uint2 nib[8];
     uint4 raw[8];                                                // fp8: the three words of chunks i, i + 1 in raw[i]
     // chunk 8h + i of a unit's block (past the block's last it re-reads that one)
-    auto request = [&](uint32_t unit, uint32_t i) {
-        const uint32_t rb = min(unit, w.units - 1u), sc = min(8u * h + i, nsc - 1u);
-        nib[i] = ldnt2(a.low + ((uint64_t)(rb * f.spr + w.cb * 16u + sc) * kLanes + L) * 8u);
+    auto request = [&](uint32_t rb, uint32_t cb, uint32_t i) {
+        const uint32_t sc = min(8u * h + i, nsc_of(cb) - 1u);
+        nib[i] = ldnt2(a.low + ((uint64_t)(rb * f.spr + cb * 16u + sc) * kLanes + L) * 8u);
         if constexpr (ELEM == kElemFp8) {
             if ((i & 1u) == 0u) {
-                const uint8_t *pp = rplane + (((uint64_t)rb * f.spr2 + w.cb * 8u + (sc >> 1)) * 3u * kLanes + L) * 4u;
+                const uint8_t *pp = rplane + (((uint64_t)rb * f.spr2 + cb * 8u + (sc >> 1)) * 3u * kLanes + L) * 4u;
                 raw[i].x = ldnt1(pp);
                 raw[i].y = ldnt1(pp + kLanes * 4u);
                 raw[i].z = ldnt1(pp + 2u * kLanes * 4u);
             }
         } else {
-            raw[i] = ldnt4(rplane + ((uint64_t)(rb * f.spr + w.cb * 16u + sc) * kLanes + L) * 16u);
+            raw[i] = ldnt4(rplane + ((uint64_t)(rb * f.spr + cb * 16u + sc) * kLanes + L) * 16u);
         }
     };
-    StageX<NT> S;
-    S.issue(p, w.cb);
+    uint32_t unit, cb;
+    w.at(w.t, unit, cb);
+    StageX S;
+    S.issue(p, w.cb0, w.direct ? f.CB : 1u);
 #pragma unroll
-    for (uint32_t i = 0; i < 8; i++) request(w.unit, i);
-    uint32_t *xs = dyn, *patch = dyn + NT * 16u * kTokensXRow + wv * kTokensPatchWords;
-    S.commit(xs, p, w.cb);
+    for (uint32_t i = 0; i < 8; i++) request(unit, cb, i);
+    constexpr uint32_t own = kTokensPatchWords + kTokensExcWords;
+    uint32_t *xs = dyn, *patch = dyn + p.xwords + w.t * own, *slot = patch + kTokensPatchWords;
+    float *sums = (float *)(dyn + p.xwords + w.step * own);
+    ExcStream<ELEM> E;
+    E.request(a, unit * f.CB + cb, a.hdr[(uint64_t)(unit * f.CB + cb) * kHdrBytes + L]);
+    uint32_t un, cn;
+    w.at(w.t + w.step, un, cn);
+    uint32_t nn = a.hdr[(uint64_t)(un * f.CB + cn) * kHdrBytes + L];
+    S.commit(xs, p);
+    E.store(slot);
     __syncthreads();
     const uint32_t r = L >> 2, q = L & 3u;
     uint32_t *wa = patch + 256u * h + 16u * r + 4u * ((q ^ (r >> 2)) & 3u);
     uint32_t *wb = patch + 256u * h + 16u * (r + 8u) + 4u * ((q ^ ((r + 8u) >> 2)) & 3u);
     const uint32_t *ra = patch + 16u * i16 + 4u * ((c4 ^ (i16 >> 2)) & 3u);
-    const uint32_t *xr = xs + i16 * kTokensXRow + 4u * c4;
-    for (; w.unit < w.units; w.unit += w.step) {
-        ExcCursor<ELEM> X;
-        X.ep = exc_start(a, w.unit * f.CB + w.cb, L, ELEM == kElemFp8 ? 2u : 3u, X.left);
+    uint32_t xr[NT];
+#pragma unroll
+    for (int j = 0; j < NT; j++) xr[j] = min(16u * j + i16, p.T - 1u) * p.xrow + 4u * c4;
+    for (; w.t < w.n; w.t += w.step) {
+        const uint32_t nsc = nsc_of(cb), *xc = xs + (w.direct ? cb * (kCols / 2u) : 0u);
+        ExcCursor<ELEM> X{(const uint8_t *)slot, E.fits ? nullptr : a.data + E.base, E.first, E.n, 0u, 0u};
+        uint32_t u2, c2;
+        w.at(w.t + 2u * w.step, u2, c2);
+        E.request(a, un * f.CB + cn, nn);
+        nn = a.hdr[(uint64_t)(u2 * f.CB + c2) * kHdrBytes + L];
         X.load();
         while (X.pos < 128u * h) X.next();                       // half 1: past the exceptions of chunks 0-7
         f32x4_t acc[NT];
@@ -523,16 +624,24 @@ __global__ void __launch_bounds__(kTokensMaxWaves * 64) k_tokens2(TokensArgs p) 
                 wave_lds_order();
                 const bf16x8_t w0 = operand(*(const uint4 *)ra), w1 = operand(*(const uint4 *)(ra + 256));
                 wave_lds_order();
-                chunk_products<NT>(w0, w1, i + 8u < nsc, xr, i, acc);
+                chunk_products<NT>(w0, w1, i + 8u < nsc, xc, xr, i, acc);
             }
-            if (ELEM != kElemFp8) request(w.unit + w.step, i);
+            if (ELEM != kElemFp8) request(un, cn, i);
             else if (i & 1u) {
-                request(w.unit + w.step, i - 1u);
-                request(w.unit + w.step, i);
+                request(un, cn, i - 1u);
+                request(un, cn, i);
             }
         }
-        store_part<NT>(p, w.cb, w.unit * 16u, acc);
+        wave_lds_order();
+        E.store(slot);
+        wave_lds_order();
+        store_part<NT, 16>(p, w, unit, sums, acc);
+        unit = un;
+        cb = cn;
+        un = u2;
+        cn = c2;
     }
+    if (w.direct) finish_direct<16>(p, w, sums);
 }
 
 // ---------------------------------------------------------------------------------------------------------------
@@ -549,7 +658,7 @@ static int launch_tokens_t(int layout, const TokensPlan &q, const TokensArgs &p,
     }
     hipLaunchKernelGGL(kernel, dim3(q.grid), dim3(q.threads), q.lds, st, p);
     e = hipGetLastError();
-    if (e != hipSuccess) return (int)e;
+    if (e != hipSuccess || p.direct) return (int)e;
     const uint64_t items = (uint64_t)p.T * (p.Mu / 4u);
     hipLaunchKernelGGL(k_tokens_finish, dim3((uint32_t)((items + 255u) / 256u)), dim3(256), 0, st, p, Shape(p.a.M, p.a.K, layout).CB);
     return (int)hipGetLastError();

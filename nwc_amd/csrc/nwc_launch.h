@@ -30,8 +30,9 @@ struct TokensArgs {
     const uint16_t *x;      // BF16 [T][ldx]
     float *part;            // sums of each column block [CB][T][Mu]
     uint32_t T, ldx, Mu;    // Mu: rows of all row groups
-    bool vec;               // K and ldx multiples of 8, x 16-byte aligned
-    uint32_t parts;         // workgroups per column block
+    uint32_t parts;         // runs of row groups: workgroups in all (direct) or per column block
+    bool direct;            // a workgroup has all column blocks of its rows and finishes them; else `part` and a second kernel
+    uint32_t xrow, xwords;  // LDS words of a token's activations (4 banks past a whole number of bank rows) and of all
     uint32_t cap;           // LDS words of a block's streams in a wave's share (layouts 0/1)
 };
 struct TokensPlan {
@@ -39,8 +40,9 @@ struct TokensPlan {
     bool seq13;
 };
 constexpr uint32_t kTokensMaxWaves = 16;
-// LDS words: a token's 512 activations (rows 4 banks apart); of a wave: layout 0's tile of exponent bytes (8 rows), layout 2's super-chunk pair
-constexpr uint32_t kTokensXRow = 260, kTokensTileRow = 132, kTokensTileWords = 8 * kTokensTileRow, kTokensPatchWords = 512;
+// LDS words of a wave: layout 0's tile of exponent bytes (8 rows, 4 banks apart), layout 2's super-chunk pair
+constexpr uint32_t kTokensTileRow = 132, kTokensTileWords = 8 * kTokensTileRow, kTokensPatchWords = 512;
+constexpr uint32_t kTokensExcWords = 256;   // a block's exceptions (fp8: 32 lanes x 7 x 2 bytes on average for Gaussian weights)
 constexpr uint32_t kTokensOverrun = 128;   // 7 super-chunks x 16 codes of at most 24 bits, and the cursor's words
 int launch_tokens(int layout, int elem_t, const TokensPlan &q, const TokensArgs &p, hipStream_t st);
 int launch_gather_fixed(int elem_t, const GatherArgs &a, hipStream_t st);

@@ -9,7 +9,7 @@ extern "C" {
 #endif
 
 /* A small batch on the matrix cores, every layout and element type: y BF16 [ntok][M] = RNE_bf16(scale * (W x[t]) + bias)
- * for 2 <= ntok <= 64, fp32 accumulation in a fixed order.  x BF16 [ntok][ldx], ldx at least K; bias BF16 [M] or null;
+ * for 2 <= ntok <= 64 and K >= 8, fp32 accumulation in a fixed order.  x BF16 [ntok][ldx], ldx at least K; bias BF16 [M] or null;
  * scale fp32 [M] or null; row_index (required for layouts 0 and 1) and seq_table (null: the stored LUT) as
  * nwc_linear_xbf16.  `ws`: 4 * ntok * Mp * CB bytes (Mp * CB: nwc_layout's out[2]) of device memory, 16-byte aligned,
  * that no other call in flight uses; its contents do not matter.  0, -1 for arguments it does not take, or a HIP error. */

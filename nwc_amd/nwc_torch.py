@@ -638,7 +638,7 @@ class NWCWeight:
     def takes_tokens(self, tokens):
         """Whether linear_tokens takes an input of this many vectors and is the fastest route for it."""
         return ((TOKENS_MIN if self.layout == 0 else 2) <= tokens <= TOKENS_MAX and self.n >= TOKENS_MIN_WEIGHTS
-                and self.in_features <= TOKENS_MAX_K and (self.layout == 2 or self.row_index() is not None))
+                and 8 <= self.in_features <= TOKENS_MAX_K and (self.layout == 2 or self.row_index() is not None))
 
     def linear_tokens(self, x: torch.Tensor, bias) -> torch.Tensor:
         """A small batch on the matrix cores without a temporary BF16 matrix, any layout: x BF16 [T, in_features], T from
