@@ -338,9 +338,9 @@ def _copy_spans(src, dst, src_start, dst_start, size, chunk=2048):
     """dst[dst_start[b] + j] = src[src_start[b] + j] for every block b and j < size[b] (all multiples of four): one kernel
     on a GPU, a chunk of blocks at a time elsewhere."""
     if src.is_cuda:
+        src_start, dst_start, size = src_start.contiguous(), dst_start.contiguous(), size.contiguous()
         with torch.cuda.device(src.device):
-            call("nwc_copy_spans", stream(), ptr(src), ptr(src_start.contiguous()), ptr(dst), ptr(dst_start.contiguous()),
-                 ptr(size.contiguous()), size.numel())
+            call("nwc_copy_spans", stream(), ptr(src), ptr(src_start), ptr(dst), ptr(dst_start), ptr(size), size.numel())
         return
     j = torch.arange(int(size.max()), device=src.device)
     for b0 in range(0, size.numel(), chunk):
@@ -366,7 +366,7 @@ class NWCWeight:
         layout = LAYOUT_DEFAULT[kind] if layout is None else int(layout)
         _check_layout(layout)
         self._shape(rows, cols, block, kind, layout)
-        if not self._encode_there(w, scale, torch.device(device)):
+        if device is None or not self._encode_there(w, scale, torch.device(device)):
             src, scale = self._source(w, kind, scale)
             stored, length, geo = _encode(src.cpu(), rows, cols, self.code)
             self._place(stored, scale, device, geo)
@@ -637,8 +637,14 @@ class NWCWeight:
 
     def takes_tokens(self, tokens):
         """Whether linear_tokens takes an input of this many vectors and is the fastest route for it."""
-        return ((TOKENS_MIN if self.layout == 0 else 2) <= tokens <= TOKENS_MAX and self.n >= TOKENS_MIN_WEIGHTS
-                and 8 <= self.in_features <= TOKENS_MAX_K and (self.layout == 2 or self.row_index() is not None))
+        if not ((TOKENS_MIN if self.layout == 0 else 2) <= tokens <= TOKENS_MAX and self.n >= TOKENS_MIN_WEIGHTS
+                and 8 <= self.in_features <= TOKENS_MAX_K):
+            return False
+        if self.layout == 2:
+            return True
+        # an index that is not there yet cannot be built during capture; the other routes need not have one
+        missing = self._row_index is None and ROW_INDEX and self.data.is_cuda and torch.cuda.is_current_stream_capturing()
+        return not missing and self.row_index() is not None
 
     def linear_tokens(self, x: torch.Tensor, bias) -> torch.Tensor:
         """A small batch on the matrix cores without a temporary BF16 matrix, any layout: x BF16 [T, in_features], T from

@@ -108,3 +108,24 @@ def test_tokens_replays(cuda):
         torch.cuda.synchronize()
         assert torch.equal(y, want)
         c.linear_tokens(x[:5].contiguous(), None)
+
+
+def test_tokens_captured_without_an_index(cuda):
+    """A matrix used with two tokens only so far has no row index; four tokens are still captured, by the batched kernel."""
+    from nwc_amd.nwc_torch import NWCLinear
+    print("tokens capture without a row index", flush=True)
+    c = _weight(2560, 1536, "bf16", 0, seed=9)
+    c._row_index = None
+    lin = NWCLinear(w=c, device="cuda")
+    x = torch.randn(4, 1536, generator=torch.Generator().manual_seed(6)).to(torch.bfloat16).cuda()
+    lin(x[:2])
+    want = c.linear_batch(x, None)
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        y = lin(x)
+    for _ in range(3):
+        y.zero_()
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(y, want)
